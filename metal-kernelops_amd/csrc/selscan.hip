@@ -1,5 +1,9 @@
 // Mamba-1 selective scan, forward and backward, for gfx950.
 //
+// Two mappings.  dstate <= 16 with groups of a multiple of 4 channels runs one lane per
+// (channel, state): fwd_lane and bwd_lane, below.  What follows is the other one, for wider
+// states and odd groups.
+//
 // Mapping: one lane per channel row (batch, d).  A wavefront holds 64 channels of
 // one (batch, group) whenever dim/ngroups is a multiple of 64 ("uniform" mode), so
 // B_t and C_t are wave-uniform and the dB/dC sums over channels are cross-lane
@@ -631,13 +635,12 @@ __global__ void __launch_bounds__(256) fwd_replay(Geo g, Ptrs p) {
 
 // ---------------------------------------------------------------- forward, lane per (channel, state)
 //
-// With dstate <= 16 and enough rows, a wavefront holds 4 channels x 16 states, lane (c, n),
-// and walks the whole sequence once, 16 steps a block: no time chunks, so no summary pass
-// and no replay.  Per block:
+// With dstate <= 16 a wavefront holds 4 channels x 16 states, lane (c, n), and walks a run of
+// the sequence, 16 steps a block.  Per block:
 //   - lane (c, n) loads step t0 + n of its channel's delta, u and z (a wavefront reads 4 rows
 //     x 16 consecutive steps) and forms that step's size and du = step * u;
 //   - the 4 channels share one (batch, group), so the block's B and C (16 states x 16 steps
-//     each) are fetched once per wavefront, 8 values a lane, and staged in LDS as float32;
+//     each) are fetched once per wavefront, 4 values of each a lane, and staged in LDS as float32;
 //   - lane (c, n) advances its one state over the 16 steps, reading step i's size and du
 //     from lane i of its row (DPP row_newbcast, folded into the multiplies) and B_n, C_n of
 //     those steps from the staged block;
@@ -645,6 +648,18 @@ __global__ void __launch_bounds__(256) fwd_replay(Geo g, Ptrs p) {
 //     (c, n) sums step t0 + n's, adds the skip, applies the gate and stores it;
 //   - the state entering the block is saved (4 channels x 16 states: 256 contiguous bytes).
 // A block's inputs are requested two blocks ahead.
+//
+// K wavefronts of a workgroup share the 4 channels and split the time (lane_chunks chooses K).
+// With K = 1 a wavefront walks the whole sequence.  With K > 1 each first advances the zero
+// state over its run (B only, no outputs), which with the run's sum of steps gives the run's
+// map x -> e^{A sum} x + drive; the maps meet in LDS, every wavefront composes those before
+// its own, and walks its run again from that entering state.  The runs cost a second pass over
+// the recurrence, but a problem of few rows has no other work for the chip: one launch in
+// place of a layout pass, a summary, a chain and a replay.
+//
+// Rows need no alignment and the length no whole blocks: elements past a row's end come from
+// the row after it or, past the last, read as zero (buffer range check), and only ever reach
+// the steps past the end, whose states nothing reads and whose outputs are not stored.
 
 template <int I, int END, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -663,89 +678,219 @@ __device__ __forceinline__ float row_newbcast(float v) {
 constexpr int kLaneChannels = 4;  // channels per wavefront in the lane-per-state kernels
 
 // One 16-step block of B and C staged through LDS for a wavefront of the lane-per-state
-// kernels, whose 4 channels share one (batch, group): lane l fetches 8 values of it (matrix
-// l / 32, state (l / 2) mod 16, steps 8 (l mod 2) ..), stages them as float32 (zeros for
-// padded states), and lane (c, n) reads its state's 16 steps back.  Rows are kBcRow floats:
-// 16-byte aligned, and the 16 rows' reads fall in distinct banks.
+// kernels, whose 4 channels share one (batch, group).  Rows are kBcRow floats: 16-byte
+// aligned, and the 16 rows' reads fall in distinct banks.
 constexpr int kBcRow = 20;
 
-template <class TU, class TB>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) fwd_lane(Geo g, Ptrs p) {
+// A raw buffer over `bytes` bytes from a wave-uniform base: loads past them return zero.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t raw_buffer(const void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), 0x00020000);
+}
+
+// The element at byte `off`, in the low bits.
+template <class T>
+__device__ __forceinline__ uint32_t buffer_word(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  if constexpr (sizeof(T) == 4)
+    return __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+  else
+    return __builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
+}
+template <class T>
+__device__ __forceinline__ float word_f32(uint32_t w) {
+  if constexpr (sizeof(T) == 4)
+    return __uint_as_float(w);
+  else
+    return to_f32(__builtin_bit_cast(T, static_cast<uint16_t>(w)));
+}
+
+// A wavefront's share of one 16-step block of B or C, staged as float32 rows of kBcRow in LDS
+// (zeros for states >= N).  VBC (16-byte aligned rows): lane l takes 4 consecutive steps of
+// state l / 4 in one access.  Otherwise it takes step l mod 16 of the states 4 e + l / 16, e =
+// 0 .. 3, so that each of its four accesses covers four 16-step runs of the wavefront (4 of
+// its own steps a lane would touch sixteen).
+template <class T, bool VBC>
+struct BcShare {
+  static constexpr int W = VBC ? static_cast<int>(sizeof(T)) : 4;
+  uint32_t w[W];
+  struct At {
+    uint32_t off[VBC ? 1 : 4];  // byte offsets in block 0
+    float* st;
+    uint32_t ok;  // bit e: share e is a state < N
+  };
+  static __device__ __forceinline__ At at(int lane, int N, int L, float* stage) {
+    At a;
+    a.ok = 0;
+    if constexpr (VBC) {
+      const int s = lane >> 2, t = 4 * (lane & 3);
+      a.ok = s < N ? 1u : 0u;
+      a.off[0] = (static_cast<uint32_t>(s < N ? s : 0) * L + t) * sizeof(T);
+      a.st = stage + s * kBcRow + t;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int s = 4 * e + (lane >> 4);
+        a.ok |= s < N ? 1u << e : 0u;
+        a.off[e] = (static_cast<uint32_t>(s < N ? s : 0) * L + (lane & 15)) * sizeof(T);
+      }
+      a.st = stage + (lane >> 4) * kBcRow + (lane & 15);
+    }
+    return a;
+  }
+  __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, const At& a, uint32_t t0) {
+    if constexpr (!VBC) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = buffer_word<T>(r, a.off[e] + t0 * sizeof(T));
+    } else if constexpr (W == 2) {
+      const mko_u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, a.off[0] + t0 * sizeof(T), 0, 0);
+      w[0] = v.x;
+      w[1] = v.y;
+    } else {
+      const mko_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, a.off[0] + t0 * sizeof(T), 0, 0);
+      w[0] = v.x;
+      w[1] = v.y;
+      w[2] = v.z;
+      w[3] = v.w;
+    }
+  }
+  // mat: 0 stages at a.st (B), 1 one matrix further (C).  left: steps of the block inside the
+  // sequence; without VBC the steps past them are staged as zeros.
+  __device__ __forceinline__ void put(const At& a, int mat, int left = HS) const {
+    float* st = a.st + mat * HS * kBcRow;
+    if constexpr (VBC) {
+      float v[4];
+      unpack_words<T, 4>(w, v);
+      *reinterpret_cast<float4*>(st) = a.ok ? make_float4(v[0], v[1], v[2], v[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        st[4 * e * kBcRow] = ((a.ok >> e) & 1u) && static_cast<int>(threadIdx.x & 15) < left ? word_f32<T>(w[e]) : 0.0f;
+    }
+  }
+};
+
+template <class TU, class TB, bool VBC, int K>
+__global__ void __launch_bounds__((K > 4 ? K : 4) * kWave) __attribute__((amdgpu_waves_per_eu(K > 4 ? 4 : 5)))
+fwd_lane(Geo g, Ptrs p) {
+  constexpr int kWaves = K > 4 ? K : 4;
   constexpr int kRow = HS + 1;   // a step's 16 states, padded so the transposed reads miss no bank
   constexpr int kCS = HS * kRow; // one channel's [step][state] block (272 floats: 16 banks apart)
-  __shared__ float sy[4][kLaneChannels * kCS];
+  __shared__ float sy[kWaves][kLaneChannels * kCS];
+  __shared__ __align__(16) float sbc[kWaves][2][HS][kBcRow];
   const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, cl = lane >> 4, n = lane & 15;
-  const int64_t row = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels + cl;
-  const bool active = row < g.rows;
-  const int64_t r = active ? row : g.rows - 1;
-  const int64_t bb = r / g.dim, d = r - bb * g.dim;
-  const int64_t bg = bb * g.ngroups + d / g.dg;
+  const int kc = wave % K;  // this wavefront's run of the sequence
+  // a wavefront's 4 rows are all valid or all past the end (4 divides the group width)
+  int64_t row0 = (static_cast<int64_t>(blockIdx.x) * (kWaves / K) + wave / K) * kLaneChannels;
+  const bool active = row0 < g.rows;
+  if (!active) row0 = g.rows - kLaneChannels;
+  const int64_t bg = uniform(static_cast<int>(row0 / g.dg));
+  const int64_t d = row0 % g.dim + cl;
   const int N = static_cast<int>(g.dstate);
   const bool sn = n < N;
   const float a2 = sn ? p.A[d * N + n] * kLog2e : 0.0f;
   const float bias = p.bias ? p.bias[d] : 0.0f;
   const float Dd = p.D ? p.D[d] : 0.0f;
   const bool has_z = p.z != nullptr;
-  const int64_t L = g.length;
-  const int64_t rbase = r * L + n;  // this lane's step of every block
-  const float* dp = static_cast<const float*>(p.delta) + rbase;
-  const TU* up = static_cast<const TU*>(p.u) + rbase;
-  const TU* zp = static_cast<const TU*>(has_z ? p.z : p.u) + rbase;
-  TU* op = static_cast<TU*>(p.out) + rbase;
-  float* sp = p.states + ck_index(g, r, 0, sn ? n : 0);
-  const int64_t sstep = g.dim * N;  // one saved state further
-  float* sw = sy[wave] + cl * kCS;
-  // The wavefront's 4 channels share one (batch, group), so one 16-step block of B and C
-  // serves all of them, staged through LDS (kBcRow).
-  __shared__ __align__(16) float sbc[4][2][HS][kBcRow];
-  const int sm = lane >> 5, sst = (lane >> 1) & 15, shf = lane & 1;
-  const bool sok = sst < N;
-  const TB* bcsrc = static_cast<const TB*>(sm ? p.C : p.B) + (bg * N + (sok ? sst : 0)) * L + 8 * shf;
-  float* stg = &sbc[wave][sm][sst][8 * shf];
+  const int L = static_cast<int>(g.length);
+  const int nblk = (L + HS - 1) / HS;
+  const int per = (nblk + K - 1) / K;
+  const int b0 = kc * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+  // the wavefront's rows of the per-element arrays, and its group's of B and C
+  constexpr uint32_t kU = sizeof(TU), kB = sizeof(TB);
+  const uint32_t rows = kLaneChannels * static_cast<uint32_t>(L);
+  const auto rdl = raw_buffer(static_cast<const float*>(p.delta) + row0 * L, rows * 4);
+  const auto ru = raw_buffer(static_cast<const TU*>(p.u) + row0 * L, rows * kU);
+  const auto rz = raw_buffer(static_cast<const TU*>(has_z ? p.z : p.u) + row0 * L, rows * kU);
+  const auto rB = raw_buffer(static_cast<const TB*>(p.B) + bg * N * L, N * static_cast<uint32_t>(L) * kB);
+  const auto rC = raw_buffer(static_cast<const TB*>(p.C) + bg * N * L, N * static_cast<uint32_t>(L) * kB);
+  const uint32_t eoff = static_cast<uint32_t>(cl) * L + n;  // this lane's step of block 0
+  const auto share = BcShare<TB, VBC>::at(lane, N, L, &sbc[wave][0][0][0]);
   const float* brow = &sbc[wave][0][n][0];
   const float* crow = &sbc[wave][1][n][0];
+  float* sw = sy[wave] + cl * kCS;
 
   struct In {
-    float dl;
-    TU u, z;
-    RawRun<TB, 8> bc;
+    uint32_t dl, u, z;
+    BcShare<TB, VBC> b, c;
   };
-  auto load = [&](int64_t t0, In& in) {
-    in.dl = dp[t0];
-    in.u = up[t0];
-    in.z = zp[t0];
-    in.bc.load(g, bcsrc, 0, t0, 8);
+  // block k's inputs; past the run's end, the last block's again
+  auto load = [&](int k, In& in, auto full) {
+    const uint32_t t0 = static_cast<uint32_t>(k < b1 ? k : b1 - 1) * HS;
+    in.dl = buffer_word<float>(rdl, (eoff + t0) * 4);
+    in.u = buffer_word<TU>(ru, (eoff + t0) * kU);
+    in.b.load(rB, share, t0);
+    if constexpr (decltype(full)::value) {
+      in.z = buffer_word<TU>(rz, (eoff + t0) * kU);
+      in.c.load(rC, share, t0);
+    }
   };
-  const int nblk = static_cast<int>(L / HS);
+  float x = 0.0f;
+  In ra, rb;
+
+  if constexpr (K > 1) {
+    // ---- the run's map, from a zero entry; the last run's is not needed
+    constexpr auto kMap = std::false_type{};
+    if (kc < K - 1 && b0 < b1) {
+      float sum = 0.0f;
+      load(b0, ra, kMap);
+      load(b0 + 1, rb, kMap);
+      auto step = [&](int k, In& in) {
+        const float del = step_of(g, __uint_as_float(in.dl), bias);
+        const float du = del * word_f32<TU>(in.u);
+        in.b.put(share, 0);
+        load(k + 2, in, kMap);
+        wave_lds_sync();
+        float bv[HS];
+        lds_row<HS>(brow, bv);
+        wave_lds_sync();
+        static_for<0, HS>([&](auto ic) {
+          constexpr int i = decltype(ic)::value;
+          x = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), x, row_newbcast<i>(du) * bv[i]);
+        });
+        sum += del;
+      };
+      for (int k = b0; k < b1; k += 2) {
+        step(k, ra);
+        if (k + 1 < b1) step(k + 1, rb);
+      }
+      sw[2 * n] = fast_exp2(a2 * row16_sum(sum));
+      sw[2 * n + 1] = x;
+    }
+    __syncthreads();
+    // the maps of the runs before this one, in order (a run with no block is past every
+    // run that has one)
+    x = 0.0f;
+    for (int j = 0; j < kc && b0 < b1; ++j) {
+      const float* m = sy[wave - kc + j] + cl * kCS + 2 * n;
+      x = fmaf(m[0], x, m[1]);
+    }
+    __syncthreads();  // the transposes take the buffers
+  }
+
+  // ---- outputs and saved states
+  if (b0 >= b1) return;
+  TU* op = static_cast<TU*>(p.out) + row0 * L + eoff;
+  const bool save = p.states != nullptr && active && sn;
+  float* sp = p.states + ck_index(g, row0, 0, 0) + (cl * N + (sn ? n : 0));
+  const int64_t sstep = g.dim * N;  // one saved state further
   // Two buffers of raw inputs: a block's raw words are unpacked first and then
   // reloaded with the block two further on (the last ones reload the last block), so
   // each load has two blocks of work to arrive.  32-bit B/C need no unpacking (the
   // raw words are the values), so their reload waits for the end of the block
   // instead of holding a second copy: one block of work, as many registers as one
   // buffer ahead.
-  auto ahead = [&](int k) { return static_cast<int64_t>(k < nblk ? k : nblk - 1) * HS; };
-  In ra, rb;
-  load(0, ra);
-  load(ahead(1), rb);
-  float x = 0.0f;
+  constexpr auto kFull = std::true_type{};
+  load(b0, ra, kFull);
+  load(b0 + 1, rb, kFull);
   auto block = [&](int k, In& in) {
-    const int64_t t0 = static_cast<int64_t>(k) * HS;
-    if (active && sn) __builtin_nontemporal_store(x, sp + k * sstep);  // whole lines, read once by the backward
-    const float uu = to_f32(in.u);
-    const float zz = to_f32(in.z);
-    const float del = step_of(g, in.dl, bias);
-    {
-      float sv[8];
-      in.bc.get(sv);
-      if (!sok) {  // a padded state adds nothing
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sv[i] = 0.0f;
-      }
-      reinterpret_cast<float4*>(stg)[0] = make_float4(sv[0], sv[1], sv[2], sv[3]);
-      reinterpret_cast<float4*>(stg)[1] = make_float4(sv[4], sv[5], sv[6], sv[7]);
-    }
-    if constexpr (sizeof(TB) == 2) load(ahead(k + 2), in);
+    const int t0 = k * HS;
+    if (save) __builtin_nontemporal_store(x, sp + k * sstep);  // whole lines, read once by the backward
+    const float uu = word_f32<TU>(in.u);
+    const float zz = word_f32<TU>(in.z);
+    const float del = step_of(g, __uint_as_float(in.dl), bias);
+    in.b.put(share, 0);
+    in.c.put(share, 1);
+    if constexpr (sizeof(TB) == 2) load(k + 2, in, kFull);
     wave_lds_sync();
     float bv[HS], cv[HS];
     lds_row<HS>(brow, bv);
@@ -765,21 +910,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) f
     wave_lds_sync();
     float y = fmaf(Dd, uu, (s4[0] + s4[1]) + (s4[2] + s4[3]));
     if (has_z) y *= zz * sigmoid(zz);
-    if (active) op[t0] = from_f32<TU>(y);
-    if constexpr (sizeof(TB) == 4) load(ahead(k + 2), in);
+    if (active && t0 + n < L) op[t0] = from_f32<TU>(y);
+    if constexpr (sizeof(TB) == 4) load(k + 2, in, kFull);
   };
-  for (int k = 0; k < nblk; k += 2) {
+  for (int k = b0; k < b1; k += 2) {
     block(k, ra);
-    if (k + 1 < nblk) block(k + 1, rb);
+    if (k + 1 < b1) block(k + 1, rb);
   }
 }
 
 // ---------------------------------------------------------------- backward, lane per (channel, state)
 //
 // The backward in fwd_lane's mapping: a wavefront holds 4 channels x 16 states, lane (c, n), and
-// walks the whole sequence once in reverse, 16 steps a block.  With every (channel, state) chain
-// on its own lane there are enough wavefronts without cutting time into chunks, so the adjoint
-// entering a block is simply carried over from the block to its right: no summary pass, no chain.
+// walks a time chunk in reverse, 16 steps a block, carrying the adjoint from each block into the
+// one on its left.  With enough rows there is one chunk, the whole sequence.  Fewer rows are cut
+// into chunks (lane_bwd_chunks): bwd_map first walks every chunk but the first with the adjoint
+// alone, from a zero exit, which with the chunk's sum of steps gives its map from the adjoint
+// entering it on the right to the one leaving it on the left; bwd_lane composes the maps of
+// the chunks to the right of its own before its first block.
 // Per block:
 //   - lane (c, n) loads step t0 + n of its channel's delta, u, z, dout and out and forms that
 //     element's step, du, gy = dout silu(z) and the factor of dz;
@@ -789,7 +937,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) f
 //     decays a = exp(A delta);
 //   - it walks the 16 steps backwards with the adjoint h_t = gy_t C_t + a_{t+1} h_{t+1}, and per
 //     step writes its state's terms of the two sums over states that du and ddelta need,
-//     h_t B_t and A a_t x_{t-1} h_t, as one pair into the wavefront's LDS transpose, and adds its
+//     h_t B_t and a_t x_{t-1} h_t, as one pair into the wavefront's LDS transpose, and adds its
 //     dA term (the adjoint and dA multiply-adds take their step's gy and delta as a DPP row
 //     broadcast, fmac_row);
 //   - the dB and dC terms, h_t du_t and gy_t x_t, are summed over the wavefront's 4 channels
@@ -799,16 +947,18 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) f
 //     exchanges odd and even rows, and one more add leaves dB_i, dB_{i+1}, dC_i and dC_{i+1} as
 //     the four rows of one register: 6 instructions per two steps, in a fixed order;
 //   - lane (c, n) then owns step t0 + n: it sums its row of the transpose and writes du,
-//     ddelta and dz.  The pre-gate output that dz needs comes back as out / silu(z); a block
-//     where silu(z) is exactly zero somewhere (or out was not given) first sums a transpose
-//     of C x instead;
+//     ddelta and dz.  The pre-gate output that dz needs comes from a transpose of C x summed
+//     over the states; with use_out it comes back as out / silu(z), except in a block where
+//     silu(z) is exactly zero somewhere;
 //   - the workgroup's 4 wavefronts add their dB/dC blocks in a fixed order and write one
 //     partial per 16 channels (per 4 channels when a group is not a multiple of 16 wide).
-// A block's inputs are requested one block ahead.  Needs dstate <= 16, whole 16-step blocks,
-// channels per group a multiple of 4, fp32 delta and 16-byte aligned rows.
+// A block's inputs are requested one block ahead.  Needs dstate <= 16, channels per group a
+// multiple of 4 and fp32 delta.  VBC: whole 16-step blocks, and 16-byte aligned rows of B and C.
+// Without it the last block's steps past the end take zeros for every input (what the loads
+// return there is the next row's, or zero past the last).
 
 // The transposes of a wavefront hold, per step, a row of 4 channels x 16 states of pairs
-// (h B, A a x h): a step's two terms leave a lane as one 8-byte write at an immediate offset
+// (h B, a x h): a step's two terms leave a lane as one 8-byte write at an immediate offset
 // from one base address.  Rows are padded to 4 mod 32 floats, so the 16-byte reads of lanes
 // (c, i..i+7), which read rows i..i+7, fall in distinct banks.
 constexpr int kTrPitch = 2 * 4 * HS + 4;
@@ -840,20 +990,96 @@ __device__ __forceinline__ float fmac_row(float acc, float v, float m) {
   return acc;
 }
 
-template <class TU, class TB>
+// One chunk's map of the adjoint: from a zero adjoint on its right, the adjoint that leaves it
+// on its left, and its sum of steps.  Chunk 0's is never needed: blockIdx.y = chunk - 1.
+template <class TU, class TB, bool VBC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) bwd_map(Geo g, Ptrs p) {
+  __shared__ __align__(16) float sbc[4][HS][kBcRow];
+  const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, cl = lane >> 4, n = lane & 15;
+  int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels;
+  const bool active = row0 < g.rows;
+  if (!active) row0 = g.rows - kLaneChannels;
+  const int64_t bg = uniform(static_cast<int>(row0 / g.dg));
+  const int64_t d = row0 % g.dim + cl;
+  const int N = static_cast<int>(g.dstate);
+  const float a2 = n < N ? p.A[d * N + n] * kLog2e : 0.0f;
+  const float bias = p.bias ? p.bias[d] : 0.0f;
+  const bool has_z = p.z != nullptr;
+  const int L = static_cast<int>(g.length);
+  const int c = blockIdx.y + 1;
+  const int nblk = (L + HS - 1) / HS, per = g.lc / HS;
+  const int b0 = c * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+  constexpr uint32_t kU = sizeof(TU);
+  const uint32_t rows = kLaneChannels * static_cast<uint32_t>(L);
+  const auto rdl = raw_buffer(static_cast<const float*>(p.delta) + row0 * L, rows * 4);
+  const auto rgo = raw_buffer(static_cast<const TU*>(p.dout) + row0 * L, rows * kU);
+  const auto rz = raw_buffer(static_cast<const TU*>(has_z ? p.z : p.dout) + row0 * L, rows * kU);
+  const auto rC = raw_buffer(static_cast<const TB*>(p.C) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
+  const uint32_t eoff = static_cast<uint32_t>(cl) * L + n;
+  const auto share = BcShare<TB, VBC>::at(lane, N, L, &sbc[wave][0][0]);
+  struct In {
+    uint32_t dl, go, z;
+    BcShare<TB, VBC> c;
+  };
+  auto load = [&](int k, In& in) {
+    const uint32_t t0 = static_cast<uint32_t>(k > b0 ? k : b0) * HS;
+    in.dl = buffer_word<float>(rdl, (eoff + t0) * 4);
+    in.go = buffer_word<TU>(rgo, (eoff + t0) * kU);
+    in.z = buffer_word<TU>(rz, (eoff + t0) * kU);
+    in.c.load(rC, share, t0);
+  };
+  In ra, rb;
+  load(b1 - 1, ra);
+  load(b1 - 2, rb);
+  float h = 0.0f, sum = 0.0f;
+  auto block = [&](int k, In& in) {
+    const int left = L - k * HS;
+    const bool ok = VBC || n < left;
+    const float del = ok ? step_of(g, __uint_as_float(in.dl), bias) : 0.0f;
+    float gy = ok ? word_f32<TU>(in.go) : 0.0f;
+    if (has_z) {
+      const float zz = ok ? word_f32<TU>(in.z) : 0.0f;
+      gy *= zz * sigmoid(zz);
+    }
+    in.c.put(share, 0, left);
+    load(k - 2, in);
+    wave_lds_sync();
+    float cv[HS];
+    lds_row<HS>(&sbc[wave][n][0], cv);
+    wave_lds_sync();
+    static_for<0, HS>([&](auto jc) {
+      constexpr int i = HS - 1 - decltype(jc)::value;
+      h = fast_exp2(row_bcast<i>(del) * a2) * fmaf(row_bcast<i>(gy), cv[i], h);
+    });
+    sum += del;
+  };
+  for (int k = b1 - 1; k >= b0; k -= 2) {
+    block(k, ra);
+    if (k > b0) block(k - 1, rb);
+  }
+  sum = row16_sum(sum);
+  if (active) {
+    const int64_t o = c * g.rows + row0 + cl;
+    p.drive[o * HS + n] = h;
+    if (n == 0) p.sumd[o] = sum;
+  }
+}
+
+template <class TU, class TB, bool VBC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-bwd_lane(Geo g, Ptrs p, int cpb) {
-  // per wavefront: the transposes of the pairs (h B, A a x h); in blocks that need it, the
+bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
+  // per wavefront: the transposes of the pairs (h B, a x h); in blocks that need it, the
   // first terms first transpose C x; the workgroup's dB/dC blocks reuse the buffers
   __shared__ __align__(16) float lds[4][kTrFloats];
   __shared__ __align__(16) float sbc[4][2][HS][kBcRow];  // B and C of the block (kBcRow)
   const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, cl = lane >> 4, n = lane & 15;
-  const int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels;  // first row of the wave
-  const bool active = row0 < g.rows;  // a wavefront's 4 rows are all valid or all past the end
-  const int64_t r = active ? row0 + cl : g.rows - 1;
-  const int64_t bb = r / g.dim, d = r - bb * g.dim;
-  const int64_t bg = uniform(static_cast<int>((active ? row0 : g.rows - 1) / g.dg));  // (batch, group) of the wave
+  const int64_t first = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels;
+  const bool active = first < g.rows;  // a wavefront's 4 rows are all valid or all past the end
+  const int64_t row0 = active ? first : g.rows - kLaneChannels;  // first row of the wave
+  const int64_t bg = uniform(static_cast<int>(row0 / g.dg));     // (batch, group) of the wave
+  const int64_t d = row0 % g.dim + cl;
   const int N = static_cast<int>(g.dstate);
   const bool sn = n < N;  // states n >= N exist only as zero lanes
   const float an = sn ? p.A[d * N + n] : 0.0f;
@@ -861,84 +1087,99 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
   const float bias = p.bias ? p.bias[d] : 0.0f;
   const float Dd = p.D ? p.D[d] : 0.0f;
   const bool has_z = p.z != nullptr;
-  const bool has_out = p.out != nullptr;
-  const int64_t L = g.length;
+  const bool has_out = use_out;
+  const int L = static_cast<int>(g.length);
   float* tr = lds[wave];
-  // Lane offsets in elements (lane_bwd_shape keeps the per-row arrays and B/C below 2^31
-  // elements each): this lane's
-  // element of a block, its saved state, and its state's row of B and C (read straight from
-  // memory: the wavefront's 4 channels read the same rows, which the vector L1 serves once).
-  // Block offsets are added to wave-uniform base pointers.
-  const uint32_t eoff = static_cast<uint32_t>(r * L + n);
-  const uint32_t soff = static_cast<uint32_t>(ck_index(g, r, 0, sn ? n : 0));
-  const int sm = lane >> 5, sst = (lane >> 1) & 15, shf = lane & 1;  // this lane's share of the B/C block
-  const bool sok = sst < N;
-  const uint32_t bcoff = static_cast<uint32_t>((bg * N + (sok ? sst : 0)) * L + 8 * shf);
-  const TB* bcsrc = static_cast<const TB*>(sm ? p.C : p.B);
-  float* stg = &sbc[wave][sm][sst][8 * shf];
+  // The wavefront's rows of the per-element arrays and its group's of B and C as buffers; this
+  // lane's element of block 0, and its share of a B/C block.
+  constexpr uint32_t kU = sizeof(TU);
+  const uint32_t rows = kLaneChannels * static_cast<uint32_t>(L);
+  const auto rdl = raw_buffer(static_cast<const float*>(p.delta) + row0 * L, rows * 4);
+  const auto ru = raw_buffer(static_cast<const TU*>(p.u) + row0 * L, rows * kU);
+  const auto rz = raw_buffer(static_cast<const TU*>(has_z ? p.z : p.u) + row0 * L, rows * kU);
+  const auto rgo = raw_buffer(static_cast<const TU*>(p.dout) + row0 * L, rows * kU);
+  const auto ro = raw_buffer(static_cast<const TU*>(has_out ? p.out : p.u) + row0 * L, rows * kU);
+  const auto rB = raw_buffer(static_cast<const TB*>(p.B) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
+  const auto rC = raw_buffer(static_cast<const TB*>(p.C) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
+  const uint32_t eoff = static_cast<uint32_t>(cl) * L + n;
+  const auto share = BcShare<TB, VBC>::at(lane, N, L, &sbc[wave][0][0][0]);
   const float* brow = &sbc[wave][0][n][0];
   const float* crow = &sbc[wave][1][n][0];
   const int tw = cl * HS + n;  // this lane's column in a transpose row
   const int64_t sstep = g.dim * N;
-  const TU* zsrc = static_cast<const TU*>(has_z ? p.z : p.u);
-  const TU* osrc = static_cast<const TU*>(has_out ? p.out : p.u);
+  const float* sbase = p.states + ck_index(g, row0, 0, 0);
+  const uint32_t soff = cl * N + (sn ? n : 0);
+  TU* duw = static_cast<TU*>(p.du) + row0 * L;
+  float* ddw = static_cast<float*>(p.ddelta) + row0 * L;
+  TU* dzw = has_z && p.dz ? static_cast<TU*>(p.dz) + row0 * L : nullptr;
   // dB/dC partial slot of the wavefront (cpb 4) or workgroup (cpb 16): partial index = first row / cpb
   float2* pbc = reinterpret_cast<float2*>(p.pbc) +
-                ((cpb == 16 ? row0 - wave * kLaneChannels : row0) / cpb) * L * HS;
+                ((cpb == 16 ? first - wave * kLaneChannels : row0) / cpb) * static_cast<int64_t>(L) * HS;
 
   struct In {
-    float dl, xin;
-    TU u, z, go, o;
-    RawRun<TB, 8> bc;
+    uint32_t dl, u, z, go, o;
+    float xin;
+    BcShare<TB, VBC> b, c;
   };
   auto load = [&](int k, In& in) {
-    const int64_t t0 = static_cast<int64_t>(k) * HS;
-    in.dl = (static_cast<const float*>(p.delta) + t0)[eoff];
-    in.u = (static_cast<const TU*>(p.u) + t0)[eoff];
-    in.z = (zsrc + t0)[eoff];
-    in.go = (static_cast<const TU*>(p.dout) + t0)[eoff];
-    in.o = (osrc + t0)[eoff];
-    in.xin = __builtin_nontemporal_load(p.states + k * sstep + soff);  // whole lines, read once
-    in.bc.load(g, bcsrc + t0, 0, bcoff, 8);
+    const uint32_t t0 = static_cast<uint32_t>(k) * HS;
+    const uint32_t e4 = (eoff + t0) * 4, eu = (eoff + t0) * kU;
+    in.dl = buffer_word<float>(rdl, e4);
+    in.u = buffer_word<TU>(ru, eu);
+    in.z = buffer_word<TU>(rz, eu);
+    in.go = buffer_word<TU>(rgo, eu);
+    in.o = buffer_word<TU>(ro, eu);
+    in.xin = __builtin_nontemporal_load(sbase + k * sstep + soff);  // whole lines, read once
+    in.b.load(rB, share, t0);
+    in.c.load(rC, share, t0);
   };
-  const int nblk = static_cast<int>(L / HS);
+  // this workgroup's chunk: blocks kb .. ke - 1
+  const int nblk = (L + HS - 1) / HS, per = g.lc / HS, ch = blockIdx.y;
+  const int kb = ch * per, ke = kb + per < nblk ? kb + per : nblk;
   In cur;
-  load(nblk - 1, cur);
+  load(ke - 1, cur);
   float carry = 0.0f;  // a_{t+1} h_{t+1} entering the block's last step from the right
-  float dA0 = 0.0f, dA1 = 0.0f, dD_acc = 0.0f, db_acc = 0.0f;  // dA in two chains (even, odd steps)
+  // the maps of the chunks to the right, fetched eight at a time (clamped: every load is issued)
+  for (int c0 = g.nchunks - 1; c0 > ch; c0 -= 8) {
+    float e[8], m[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t o = (c0 - q > ch ? c0 - q : ch + 1) * g.rows + row0 + cl;
+      e[q] = p.sumd[o];
+      m[q] = p.drive[o * HS + n];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (c0 - q > ch) carry = fmaf(fast_exp2(a2 * e[q]), carry, m[q]);
+  }
+  float dA_acc = 0.0f, dD_acc = 0.0f, db_acc = 0.0f;
   const float act = active ? 1.0f : 0.0f;
 
-  for (int k = nblk - 1; k >= 0; --k) {
-    const int64_t t0 = static_cast<int64_t>(k) * HS;
+  for (int k = ke - 1; k >= kb; --k) {
+    const int t0 = k * HS;
+    const int left = L - t0;
+    const bool ok = VBC || n < left;
     // ---- this lane's element: step t0 + n of channel c
-    const float uu = to_f32(cur.u);
-    const float del = step_of(g, cur.dl, bias);
+    const float uu = ok ? word_f32<TU>(cur.u) : 0.0f;
+    const float del = ok ? step_of(g, __uint_as_float(cur.dl), bias) : 0.0f;
     const float du = del * uu;
-    float gy = to_f32(cur.go) * act;
+    float gy = ok ? word_f32<TU>(cur.go) * act : 0.0f;
     float dzf = 0.0f, ypre = 0.0f;
     bool need_y = false;
     if (has_z) {
-      const float zz = to_f32(cur.z);
+      const float zz = ok ? word_f32<TU>(cur.z) : 1.0f;
       const float sg = sigmoid(zz);
       const float gate = zz * sg;
       dzf = gy * sg * (1.0f + zz * (1.0f - sg));
-      if (has_out && gate != 0.0f) ypre = to_f32(cur.o) * fast_rcp(gate);
+      if (has_out && gate != 0.0f) ypre = word_f32<TU>(cur.o) * fast_rcp(gate);
       else need_y = true;
       gy *= gate;
     }
     const bool ty = __ballot(need_y) != 0;  // wave-uniform: transpose C x in this block
     const float x0 = sn ? cur.xin : 0.0f;
-    {
-      float sv[8];
-      cur.bc.get(sv);
-      if (!sok) {  // a padded state adds nothing
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sv[i] = 0.0f;
-      }
-      reinterpret_cast<float4*>(stg)[0] = make_float4(sv[0], sv[1], sv[2], sv[3]);
-      reinterpret_cast<float4*>(stg)[1] = make_float4(sv[4], sv[5], sv[6], sv[7]);
-    }
-    load(k > 0 ? k - 1 : 0, cur);  // the next block's inputs: a block of work to arrive
+    cur.b.put(share, 0, left);
+    cur.c.put(share, 1, left);
+    load(k > kb ? k - 1 : kb, cur);  // the next block's inputs: a block of work to arrive
     wave_lds_sync();
     float bv[HS], cv[HS];
     lds_row<HS>(brow, bv);
@@ -971,6 +1212,7 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
       recompute(std::false_type{});
     }
     // ---- reverse walk
+    float dA0, dA1;  // the block's dA in two chains (even, odd steps)
     float sbc[HS / 2];  // dB/dC of step pairs summed over the wavefront's 4 channels (see below)
     float rodd = 0.0f;  // the odd step's half-summed register, waiting for its even partner
     static_for<0, HS>([&](auto jc) {
@@ -978,8 +1220,10 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
       const float h = fmac_row<i, i == HS - 1>(carry, gy, cv[i]);
       const float hc = ah[i] * h;
       const float pr = hc * (i > 0 ? xh[i > 0 ? i - 1 : 0] : x0);
-      *reinterpret_cast<float2*>(tr + i * kTrPitch + 2 * tw) = make_float2(h * bv[i], an * pr);
-      if constexpr (i % 2 == 0) dA0 = fmac_row<i>(dA0, del, pr);
+      *reinterpret_cast<float2*>(tr + i * kTrPitch + 2 * tw) = make_float2(h * bv[i], pr);
+      if constexpr (i == HS - 1) dA1 = row_bcast<i>(del) * pr;
+      else if constexpr (i == HS - 2) dA0 = row_bcast<i>(del) * pr;
+      else if constexpr (i % 2 == 0) dA0 = fmac_row<i>(dA0, del, pr);
       else dA1 = fmac_row<i>(dA1, del, pr);
       // dB and dC terms of step i, h du_i and gy_i x_i: rows c0 + c2 and c1 + c3 of each
       // (a swap of the wavefront's halves), dB in rows 0-1 and dC in rows 2-3 ...
@@ -996,23 +1240,20 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
       }
       carry = hc;
     });
+    dA_acc += dA0 + dA1;
     wave_lds_sync();
     // ---- lane (c, n) owns step t0 + n: its row of the transpose
     float s1, s2;
     {
       float v[2 * HS];
       lds_row<2 * HS>(tr + n * kTrPitch + 2 * cl * HS, v);
-      float a[4], b[4];
-#pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        a[m] = v[2 * m];
-        b[m] = v[2 * m + 1];
-      }
-#pragma unroll
-      for (int m = 4; m < HS; ++m) {
+      // the second sum's factor A of state m comes from lane m of the row: one rounding a term
+      float a[4] = {}, b[4] = {};
+      static_for<0, HS>([&](auto mc) {
+        constexpr int m = decltype(mc)::value;
         a[m & 3] += v[2 * m];
-        b[m & 3] += v[2 * m + 1];
-      }
+        b[m & 3] = fmaf(row_bcast<m>(an), v[2 * m + 1], b[m & 3]);
+      });
       s1 = (a[0] + a[1]) + (a[2] + a[3]);
       s2 = (b[0] + b[1]) + (b[2] + b[3]);
     }
@@ -1021,10 +1262,10 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
     if (g.softplus) dd *= softplus_grad_from_value(del);
     dD_acc = fmaf(gy, uu, dD_acc);
     db_acc = fmaf(dd, act, db_acc);
-    if (active) {
-      (static_cast<TU*>(p.du) + t0)[eoff] = from_f32<TU>(duo);
-      (static_cast<float*>(p.ddelta) + t0)[eoff] = dd;
-      if (has_z && p.dz) (static_cast<TU*>(p.dz) + t0)[eoff] = from_f32<TU>(dzf * ypre);
+    if (active && ok) {
+      duw[eoff + t0] = from_f32<TU>(duo);
+      ddw[eoff + t0] = dd;
+      if (dzw) dzw[eoff + t0] = from_f32<TU>(dzf * ypre);
     }
     // ---- dB/dC of the block: register m of lane (row q, state n) holds dB (q < 2) or dC (q >= 2)
     // of step 2m + (q mod 2)
@@ -1042,26 +1283,27 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
         sb += lds[w][o];
         sc += lds[w][HS * HS + o];
       }
-      {
+      if (VBC || o / HS < left) {
         // whole 2 KB runs that only reduce_bc reads back: written with the nontemporal hint
         // (the per-lane element streams above keep plain accesses: a wavefront covers half a
         // line of each per block, and the next block uses the other half)
         const mko_u32x2 w = {__float_as_uint(sb), __float_as_uint(sc)};
-        __builtin_nontemporal_store(w, reinterpret_cast<mko_u32x2*>(pbc + t0 * HS) + o);
+        __builtin_nontemporal_store(w, reinterpret_cast<mko_u32x2*>(pbc + static_cast<int64_t>(t0) * HS) + o);
       }
       __syncthreads();
     } else if (active) {
-      float* pf = reinterpret_cast<float*>(pbc + t0 * HS) + which;
+      float* pf = reinterpret_cast<float*>(pbc + static_cast<int64_t>(t0) * HS) + which;
 #pragma unroll
-      for (int m = 0; m < HS / 2; ++m) pf[((2 * m + par) * HS + n) * 2] = sbc[m];
+      for (int m = 0; m < HS / 2; ++m)
+        if (VBC || 2 * m + par < left) pf[((2 * m + par) * HS + n) * 2] = sbc[m];
     }
   }
-  if (active && sn) p.dap[static_cast<int64_t>(n) * g.rows + row0 + cl] = dA0 + dA1;
+  if (active && sn) p.dap[(static_cast<int64_t>(ch) * HS + n) * g.rows + row0 + cl] = dA_acc;
   dD_acc = row16_sum(dD_acc);
   db_acc = row16_sum(db_acc);
   if (active && n == 0) {
-    p.ddp[row0 + cl] = dD_acc;
-    p.dbp[row0 + cl] = db_acc;
+    p.ddp[ch * g.rows + row0 + cl] = dD_acc;
+    p.dbp[ch * g.rows + row0 + cl] = db_acc;
   }
 }
 
@@ -1498,7 +1740,7 @@ __global__ void __launch_bounds__(256) reduce_bc(Geo g, int ncb, int64_t seg_dg,
     const int64_t t = t0 + tl;
     float vb = 0.0f, vc = 0.0f;
     if (t < g.length) {
-      // channel blocks in order: whole batches of sixteen issue their loads together, the
+      // channel blocks in a fixed order: whole batches of sixteen issue their loads together, the
       // rest one at a time; the partials are read once, with the nontemporal hint (eight at a
       // time without it: 0.135 ms at c3; sixteen with it: 0.107 ms, thirty-two the same)
       constexpr int PF = 16;
@@ -1509,11 +1751,22 @@ __global__ void __launch_bounds__(256) reduce_bc(Geo g, int ncb, int64_t seg_dg,
         uint32_t q[PF][2];
 #pragma unroll
         for (int j = 0; j < PF; ++j) load_words_nt(src + (cbk + j) * stride, q[j]);
+        // pairwise inside a batch: a sum over hundreds of partials keeps its last digits
+        float b[PF], c[PF];
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
-          vb += __uint_as_float(q[j][0]);
-          vc += __uint_as_float(q[j][1]);
+          b[j] = __uint_as_float(q[j][0]);
+          c[j] = __uint_as_float(q[j][1]);
         }
+#pragma unroll
+        for (int w = PF / 2; w >= 1; w >>= 1)
+#pragma unroll
+          for (int j = 0; j < w; ++j) {
+            b[j] += b[j + w];
+            c[j] += c[j + w];
+          }
+        vb += b[0];
+        vc += c[0];
       }
       for (; cbk < nsum; ++cbk) {
         uint32_t q[2];
@@ -1614,13 +1867,14 @@ struct Plan {
   int ns;
   bool uni;
   bool lane;  // forward through fwd_lane (set per call from pointer alignment and shape)
+  bool vbc;   // fwd_lane reads B and C as vectors
   bool lane_bwd;  // backward through bwd_lane (likewise)
   size_t off_bt, off_ct, off_bn, off_cn, off_drive, off_sumd, off_adj, off_pbc, off_dap, off_ddp,
       off_dbp;
   // bwd_lane's workspace: dB/dC partials per cpb channels, dA / dD / ddelta_bias partials per row
-  int cpb;
+  int cpb, lchunks;
   int64_t lncb;
-  size_t loff_pbc, loff_dap, loff_ddp, loff_dbp;
+  size_t loff_pbc, loff_dap, loff_ddp, loff_dbp, loff_drive, loff_sumd;
   size_t fwd_bytes, bwd_bytes;
 };
 
@@ -1628,13 +1882,42 @@ inline size_t align_up(size_t v) { return (v + 255) & ~static_cast<size_t>(255);
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Rows from which the lane-per-state kernels have enough wavefronts (rows / 4 of them) to fill
-// the chip without time chunks.
+// Rows from which one wavefront per 4 of them fills the chip without time chunks.
 constexpr int64_t kLaneRows = 6144;
 
 // Shapes the lane-per-state forward takes (dtypes and alignment are checked per call).
+// Its buffers over 4 rows, and over a group's B or C, hold fewer than 2^32 bytes.
 static bool lane_shape(const Geo& g, int ns) {
-  return ns == 16 && g.rows >= kLaneRows && g.length % HS == 0 && g.dg % kLaneChannels == 0;
+  return ns == 16 && g.dg % kLaneChannels == 0 && g.d_dtype == MKO_F32 && g.length < (1 << 26);
+}
+
+// Wavefronts that share 4 channels and split the time in fwd_lane (rows / 4 quads of them).  A
+// split costs a second pass over the recurrence and pays while one wavefront per quad leaves
+// SIMDs (1024) idle or unevenly loaded.  us a forward with 1 / 4 / 16, bf16: 5120 rows x 1024
+// steps 57 / 46 / 63, 1536 x 2048 82 / 45 / 43, 384 x 3136 122 / 47 / 33; 2 x 3072 rows x 748
+// are even (46 / 44 / 63), and at 8 x 1536 x 2048 the split loses (150 / 199 / 257).
+static int lane_chunks(const Geo& g) {
+  const int64_t quads = g.rows / kLaneChannels;
+  const int64_t nblk = (g.length + HS - 1) / HS;
+  if (quads >= 1536 || nblk < 4) return 1;
+  return quads <= 384 && nblk >= 32 ? 16 : 4;
+}
+
+// Time chunks of the lane-per-state backward: the smallest power of two that gives every slot
+// of the chip (3 wavefronts on each of 1024 SIMDs) a wavefront, with at least four blocks each.
+// A chunk costs its bwd_map and its own dA / dD / ddelta_bias partials.  us a backward with
+// 1 / 2 / 4 / 8 / 32 chunks, bf16: 5120 rows x 1024 steps 153 / 131 / 116 / 117 / 149, 1536 x 2048
+// 210 / 141 / 101 / 78 / 84, 384 x 3136 309 / 199 / 110 / 67 / 48, 8 x 1536 x 2048 413 / 436.
+static int lane_bwd_chunks(const Geo& g) {
+  const int64_t quads = g.rows / kLaneChannels;
+  const int64_t nblk = (g.length + HS - 1) / HS;
+  int64_t k = 1;
+  // Steps taken as they are carry no softplus rounding, and ddelta then shows that of the decays'
+  // products along a chunk (2.1e-7 of it over 112 steps, 1.75e-7 over 64): chunks half as long.
+  const int64_t slots = g.softplus ? 3072 : 6144;
+  while (k < slots / 96 && quads * k < slots && nblk >= 8 * k) k <<= 1;
+  const int64_t per = (nblk + k - 1) / k;
+  return static_cast<int>((nblk + per - 1) / per);
 }
 
 // The backward's too.  It indexes the per-row arrays (u, delta, z, dout, out, du, ddelta, dz,
@@ -1740,11 +2023,15 @@ static int make_plan(const mko_selscan_params* p, Plan* pl) {
   pl->cpb = (g.dg % 16) == 0 ? 16 : 4;
   pl->lncb = g.dg / pl->cpb;
   if (lane_bwd_shape(g, pl->ns)) {
+    pl->lchunks = g.length > 0 ? lane_bwd_chunks(g) : 1;
+    const size_t rch = static_cast<size_t>(g.rows) * pl->lchunks;
     size_t q = 0;
     pl->loff_pbc = q; q = align_up(q + static_cast<size_t>(g.batch * g.ngroups) * pl->lncb * g.length * 16 * 2 * 4);
-    pl->loff_dap = q; q = align_up(q + static_cast<size_t>(g.rows) * 16 * 4);
-    pl->loff_ddp = q; q = align_up(q + static_cast<size_t>(g.rows) * 4);
-    pl->loff_dbp = q; q = align_up(q + static_cast<size_t>(g.rows) * 4);
+    pl->loff_dap = q; q = align_up(q + rch * 16 * 4);
+    pl->loff_ddp = q; q = align_up(q + rch * 4);
+    pl->loff_dbp = q; q = align_up(q + rch * 4);
+    pl->loff_drive = q; q = align_up(q + rch * 16 * 4);
+    pl->loff_sumd = q; q = align_up(q + rch * 4);
     if (q > pl->bwd_bytes) pl->bwd_bytes = q;
   }
   return MKO_OK;
@@ -1802,25 +2089,35 @@ static bool chain_by_wave(const Geo& g) {
 }
 
 
+template <class TU, class TB, bool VBC>
+static void launch_fwd_lane_t(const Geo& g, int k, const Ptrs& q, hipStream_t s) {
+  const int64_t quads = g.rows / kLaneChannels;
+  if (k == 1)
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1><<<blocks_for(quads, 4), 256, 0, s>>>(g, q));
+  else if (k == 4)
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4><<<blocks_for(quads, 1), 256, 0, s>>>(g, q));
+  else
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16><<<blocks_for(quads, 1), 1024, 0, s>>>(g, q));
+}
+
 template <class TU>
 static int launch_fwd_lane(const Plan& pl, const Ptrs& q, hipStream_t s) {
   const Geo& g = pl.g;
-  const unsigned grid = static_cast<unsigned>((g.rows + 4 * kLaneChannels - 1) / (4 * kLaneChannels));
-  if (g.bc_dtype == MKO_BF16)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, bf16><<<grid, 256, 0, s>>>(g, q));
-  else if (g.bc_dtype == MKO_F16)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, _Float16><<<grid, 256, 0, s>>>(g, q));
-  else
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, float><<<grid, 256, 0, s>>>(g, q));
+  const int k = lane_chunks(g);
+  auto go = [&](auto tb) {
+    using TB = decltype(tb);
+    if (pl.vbc) launch_fwd_lane_t<TU, TB, true>(g, k, q, s);
+    else launch_fwd_lane_t<TU, TB, false>(g, k, q, s);
+  };
+  if (g.bc_dtype == MKO_BF16) go(bf16{});
+  else if (g.bc_dtype == MKO_F16) go(_Float16{});
+  else go(float{});
   return mko_check_launch("selscan_fwd");
 }
 
 template <int NS, bool UNI, class TU>
 static int launch_fwd(const Plan& pl, const Ptrs& q, hipStream_t s) {
   const Geo& g = pl.g;
-  if constexpr (NS == 16 && !__is_same(TU, Dyn)) {
-    if (pl.lane) return launch_fwd_lane<TU>(pl, q, s);
-  }
   const dim3 block(g.wpg * kWave);
   const unsigned gx = static_cast<unsigned>((g.nwr + g.wpg - 1) / g.wpg);
   const int64_t ntiles = (g.length + kPrepSteps - 1) / kPrepSteps;
@@ -1851,15 +2148,32 @@ static int launch_bwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_par
   q.dap = reinterpret_cast<float*>(ws + pl.loff_dap);
   q.ddp = reinterpret_cast<float*>(ws + pl.loff_ddp);
   q.dbp = reinterpret_cast<float*>(ws + pl.loff_dbp);
-  const unsigned grid = static_cast<unsigned>((g.rows + 4 * kLaneChannels - 1) / (4 * kLaneChannels));
-  if (g.bc_dtype == MKO_BF16)
-    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, bf16><<<grid, 256, 0, s>>>(g, q, pl.cpb));
-  else if (g.bc_dtype == MKO_F16)
-    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, _Float16><<<grid, 256, 0, s>>>(g, q, pl.cpb));
-  else
-    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, float><<<grid, 256, 0, s>>>(g, q, pl.cpb));
-  // partials: dB/dC per cpb channels; dA / dD / ddelta_bias per row (one "chunk")
-  g.nchunks = 1;
+  q.drive = reinterpret_cast<float*>(ws + pl.loff_drive);
+  q.sumd = reinterpret_cast<float*>(ws + pl.loff_sumd);
+  g.nchunks = pl.lchunks;
+  const int64_t nblk = (g.length + HS - 1) / HS;
+  g.lc = static_cast<int>((nblk + g.nchunks - 1) / g.nchunks) * HS;
+  const unsigned gx = blocks_for(g.rows, 4 * kLaneChannels);
+  // Taking the pre-gate output back from the rounded out adds that rounding to dz (2.3e-3 against
+  // 2.0e-3 in bf16), so only the problems that fill the chip by themselves and are bound by vector
+  // issue do it, whole blocks of at least kLaneRows rows (4 x 5120 x 4096
+  // 1325 us against 1503 with the sum, 8 x 1536 x 2048 386 against 460).
+  const bool use_out = q.out != nullptr && g.rows >= kLaneRows;
+  auto go = [&](auto tb, auto vbc) {
+    using TB = decltype(tb);
+    constexpr bool VBC = decltype(vbc)::value;
+    if (g.nchunks > 1)
+      MKO_TIMED("selscan_bwd_map", s, bwd_map<TU, TB, VBC><<<dim3(gx, g.nchunks - 1), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, TB, VBC><<<dim3(gx, g.nchunks), 256, 0, s>>>(g, q, pl.cpb, VBC && use_out));
+  };
+  auto go_b = [&](auto tb) {
+    if (pl.vbc && g.length % HS == 0) go(tb, std::true_type{});
+    else go(tb, std::false_type{});
+  };
+  if (g.bc_dtype == MKO_BF16) go_b(bf16{});
+  else if (g.bc_dtype == MKO_F16) go_b(_Float16{});
+  else go_b(float{});
+  // partials: dB/dC per cpb channels; dA / dD / ddelta_bias per row and chunk
   MKO_TIMED("selscan_bwd_reduce", s,
             reduce_bc<16><<<static_cast<unsigned>(g.batch * g.ngroups * ((g.length + 256 / 16 - 1) / (256 / 16))),
                             256, 0, s>>>(g, static_cast<int>(pl.lncb), 0, q.pbc, p->dB, p->dC);
@@ -1870,9 +2184,6 @@ static int launch_bwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_par
 
 template <int NS, bool UNI, class TU>
 static int launch_bwd(const Plan& pl, const Ptrs& q, const mko_selscan_params* p, hipStream_t s) {
-  if constexpr (NS == 16 && !__is_same(TU, Dyn)) {
-    if (pl.lane_bwd) return launch_bwd_lane<TU>(pl, q, p, s);
-  }
   const Geo& g = pl.g;
   const dim3 block(g.wpg * kWave);
   const unsigned gx = static_cast<unsigned>((g.nwr + g.wpg - 1) / g.wpg);
@@ -1959,10 +2270,15 @@ extern "C" int mko_selscan_fwd(const mko_selscan_params* p, void* stream) {
   }
   pl.g.vec = rows_vectorisable(pl.g, {{p->u, p->u_dtype}, {p->delta, p->delta_dtype}, {p->z, p->u_dtype},
                                       {p->out, p->u_dtype}}) ? 1 : 0;
-  pl.lane = lane_shape(pl.g, pl.ns) &&
-            rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
+  pl.lane = lane_shape(pl.g, pl.ns);
+  pl.vbc = rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
   Ptrs q = make_ptrs(p, pl);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (pl.lane) {
+    if (p->u_dtype == MKO_BF16) return launch_fwd_lane<bf16>(pl, q, s);
+    if (p->u_dtype == MKO_F16) return launch_fwd_lane<_Float16>(pl, q, s);
+    return launch_fwd_lane<float>(pl, q, s);
+  }
   return dispatch_types(pl, p->u_dtype, p->delta_dtype, [&](auto tag) {
     using TU = decltype(tag);
     if (pl.ns == 16) return pl.uni ? launch_fwd<16, true, TU>(pl, q, s) : launch_fwd<16, false, TU>(pl, q, s);
@@ -1990,9 +2306,15 @@ extern "C" int mko_selscan_bwd(const mko_selscan_params* p, void* stream) {
   pl.g.vec = rows_vectorisable(pl.g, {{p->u, p->u_dtype}, {p->delta, p->delta_dtype}, {p->z, p->u_dtype},
                                       {p->dout, p->u_dtype}, {p->du, p->u_dtype}, {p->ddelta, p->delta_dtype},
                                       {p->dz, p->u_dtype}, {p->out, p->u_dtype}}) ? 1 : 0;
-  pl.lane_bwd = lane_bwd_shape(pl.g, pl.ns) && rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
+  pl.lane_bwd = lane_bwd_shape(pl.g, pl.ns);
+  pl.vbc = rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
   Ptrs q = make_ptrs(p, pl);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (pl.lane_bwd) {
+    if (p->u_dtype == MKO_BF16) return launch_bwd_lane<bf16>(pl, q, p, s);
+    if (p->u_dtype == MKO_F16) return launch_bwd_lane<_Float16>(pl, q, p, s);
+    return launch_bwd_lane<float>(pl, q, p, s);
+  }
   return dispatch_types(pl, p->u_dtype, p->delta_dtype, [&](auto tag) {
     using TU = decltype(tag);
     if (pl.ns == 16) return pl.uni ? launch_bwd<16, true, TU>(pl, q, p, s) : launch_bwd<16, false, TU>(pl, q, p, s);

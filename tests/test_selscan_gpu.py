@@ -360,3 +360,43 @@ def test_errors():
     y = scan_mps(*gpu)
     ref = oracle.selective_scan(*cpu)
     assert max_rel(y, ref) <= 1e-5
+
+
+# (batch, dim, length, dstate, groups): a single step; one step short of, at and past a 16-step
+# block; the lengths at which the forward splits the time over 4 and over 16 wavefronts, with a
+# last run of one ragged block and with runs that hold none; backward chunks of 4 blocks and a
+# short last one; groups of 4 and of 16 channels; padded states; rows that are not a multiple of
+# 16 bytes.
+SPLIT_SHAPES = [(1, 4, 1, 16, 1), (2, 8, 15, 16, 2), (1, 16, 17, 5, 1), (1, 12, 49, 16, 3), (2, 16, 511, 16, 1),
+                (1, 8, 529, 8, 2), (1, 4, 1043, 16, 1), (3, 48, 520, 16, 1)]
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16, torch.float16], ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("shape", SPLIT_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_lane_time_splits_and_ragged_rows(shape, act):
+    inputs, dy = _random_problem(*shape, seed=sum(shape) + 7, act=act)
+    assert "selscan_fwd_lane" in _forward_kernels(inputs, True)
+    assert "selscan_bwd_lane" in _backward_kernels(inputs, dy)
+    _compare(inputs, dy, True, "split " + "x".join(map(str, shape)) + f" {act}")
+
+
+@pytest.mark.parametrize("length", [37, 531])
+def test_ragged_rows_keep_apart(length):
+    # A ragged row's last block reads on into the next row: nothing of it may come back.  Channel 5
+    # is NaN throughout, and so are B's and C's last states; every other channel must match a run
+    # without them.
+    inputs, dy = _random_problem(1, 8, length, 16, 2, seed=3)
+    clean = _gpu(inputs, dy, True)
+    bad = {k: v.clone() for k, v in inputs.items()}
+    for k in ("u", "dt", "z"):
+        bad[k][0, 5] = float("nan")
+    for k in ("B", "C"):
+        bad[k][0, 1] = float("nan")
+    out, grads = _gpu(bad, dy, True)
+    assert torch.equal(out[:, :4], clean[0][:, :4])
+    for k in ("u", "dt", "z"):
+        assert torch.equal(grads[k][:, :4], clean[1][k][:, :4]), k
+    for k in ("B", "C"):
+        assert torch.equal(grads[k][:, 0], clean[1][k][:, 0]), k
+    for k in ("A", "D", "delta_bias"):
+        assert torch.equal(grads[k][:4], clean[1][k][:4]), k
