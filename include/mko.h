@@ -137,9 +137,8 @@ int mko_selscan_fwd(const mko_selscan_params* p, void* stream);
 size_t mko_selscan_bwd_workspace_size(const mko_selscan_params* p);
 int mko_selscan_bwd(const mko_selscan_params* p, void* stream);
 
-/* Which mapping each direction takes for this geometry, from the sizes alone (a call
- * still falls back to the lane-per-channel kernels when B/C rows are not 16-byte
- * aligned): 1 for the lane-per-(channel, state) kernels, 0 for the lane-per-channel ones.
+/* Which mapping each direction takes for this geometry: 1 for the lane-per-(channel, state)
+ * kernels, 0 for the lane-per-channel ones.
  * Host only, no launch; pointers are not read.  No reference counterpart (the reference
  * has one Metal mapping). */
 int mko_selscan_plan(const mko_selscan_params* p, int* fwd_lane, int* bwd_lane);
@@ -317,6 +316,12 @@ int mko_path_stack(const mko_path_params* p, void* stream);
  * in its permuting form; the reference's forward merges per-pixel slices, this
  * build's forward merges step-ordered ones like its backward. */
 int mko_path_merge(const mko_path_params* p, void* stream);
+
+/* The same for p[0 .. count), at most MKO_PATH_MAPS maps of any sizes and dtypes, in one
+ * launch: the inputs of one 2D scan, or its gradients. */
+#define MKO_PATH_MAPS 4
+int mko_path_stack_many(const mko_path_params* p, int count, void* stream);
+int mko_path_merge_many(const mko_path_params* p, int count, void* stream);
 
 /* ======================================================================== */
 /* Causal depthwise conv1d (cv/causal_conv1d.py)                              */

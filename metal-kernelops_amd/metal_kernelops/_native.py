@@ -131,6 +131,8 @@ _SIGNATURES = {
     "mko_sizeof_path_params": ([], ctypes.c_size_t),
     "mko_path_stack": ([ctypes.POINTER(PathParams), _vp], ctypes.c_int),
     "mko_path_merge": ([ctypes.POINTER(PathParams), _vp], ctypes.c_int),
+    "mko_path_stack_many": ([ctypes.POINTER(PathParams), ctypes.c_int, _vp], ctypes.c_int),
+    "mko_path_merge_many": ([ctypes.POINTER(PathParams), ctypes.c_int, _vp], ctypes.c_int),
     "mko_sizeof_conv1d_params": ([], ctypes.c_size_t),
     "mko_sizeof_conv1d_update_params": ([], ctypes.c_size_t),
     "mko_conv1d_fwd": ([ctypes.POINTER(Conv1dParams), _vp], ctypes.c_int),

@@ -12,11 +12,11 @@ state and no skip, gate or bias, and the four results are added at every pixel
 
 How it runs: the four paths of every channel are one Mamba-1 problem with four times
 the channels and groups.  ``mko::path_stack`` (a HIP gather) writes u, dt, B and C in
-path-step order, ``mko::selscan_fwd`` scans the stacked rows with the same kernels as
+path-step order in one launch, ``mko::selscan_fwd`` scans the stacked rows with the same kernels as
 ``selective_scan``, and ``mko::path_merge`` (a HIP gather) adds the four step-ordered
 slices back per pixel in the reference's ``(0 + 2) + (1 + 3)`` order.  The backward
 re-stacks the inputs and the output gradient, runs ``mko::selscan_bwd`` on the stacked
-problem, and folds du, ddt, dB and dC back with ``path_merge``; dA sums the four
+problem, and folds du, ddt, dB and dC back with one ``path_merge`` launch; dA sums the four
 paths.  The reference stacks for its backward in the same way (``:477-543``) and
 walks the paths with a cursor in its forward; here both directions share the 1-D
 scan's kernels and their deterministic dB/dC reductions.
@@ -95,30 +95,39 @@ def _zero_result(shape, tensors):
 # --------------------------------------------------------------------------- layout ops
 
 
-def _path_call(fn, x, out, height, width, scale):
-    p = nat.PathParams()
-    p.src, p.dst = x.data_ptr(), out.data_ptr()
-    p.batch, p.height, p.width = x.shape[0], height, width
-    p.rows = out.shape[1] if fn == "mko_path_merge" else x.shape[1]
-    p.dtype, p.scale = nat.code(x.dtype), float(scale)
-    lib = nat.lib()
-    nat.check(getattr(lib, fn)(ctypes.byref(p), nat.stream_of(x.device)), fn)
+def _path_call(fn, xs, outs, height, width, scale):
+    """One launch over the maps ``xs`` into ``outs`` (the library's limit is four)."""
+    params = (nat.PathParams * len(xs))()
+    for p, x, out in zip(params, xs, outs):
+        p.src, p.dst = x.data_ptr(), out.data_ptr()
+        p.batch, p.height, p.width = x.shape[0], height, width
+        p.rows = min(x.shape[1], out.shape[1])
+        p.dtype, p.scale = nat.code(x.dtype), scale
+    nat.check(getattr(nat.lib(), fn)(params, len(xs), nat.stream_of(xs[0].device)), fn)
+
+
+def _stack_all(xs, height, width, scale):
+    """Each (batch, rows, H*W) -> (batch, 4 rows, H*W): the four paths in step order."""
+    outs = [x.new_empty(x.shape[0], 4 * x.shape[1], x.shape[2]) for x in xs]
+    _path_call("mko_path_stack_many", xs, outs, height, width, float(scale))
+    return outs
+
+
+def _merge_all(xs, height, width, scale):
+    """Each (batch, 4 rows, H*W) in step order -> (batch, rows, H*W) per pixel."""
+    outs = [x.new_empty(x.shape[0], x.shape[1] // 4, x.shape[2]) for x in xs]
+    _path_call("mko_path_merge_many", xs, outs, height, width, float(scale))
+    return outs
 
 
 def _stack_impl(x: Tensor, height: int, width: int, scale: float) -> Tensor:
-    """(batch, rows, H*W) -> (batch, 4 rows, H*W): the four paths in step order."""
-    out = x.new_empty(x.shape[0], 4 * x.shape[1], x.shape[2])
-    if out.numel():
-        _path_call("mko_path_stack", x, out, height, width, scale)
-    return out
+    """One map of :func:`_stack_all`."""
+    return _stack_all([x], height, width, scale)[0]
 
 
 def _merge_impl(x: Tensor, height: int, width: int, scale: float) -> Tensor:
-    """(batch, 4 rows, H*W) in step order -> (batch, rows, H*W) per pixel."""
-    out = x.new_empty(x.shape[0], x.shape[1] // 4, x.shape[2])
-    if out.numel():
-        _path_call("mko_path_merge", x, out, height, width, scale)
-    return out
+    """One map of :func:`_merge_all`."""
+    return _merge_all([x], height, width, scale)[0]
 
 
 # The layout launches as torch ops; the 2D scan's own autograd function calls the
@@ -143,11 +152,9 @@ def _stacked(u, dt, A, B, C):
     batch, channels, height, width = u.shape
     groups, states = B.shape[1], A.shape[1]
     length = height * width
-    stack = _stack_impl
-    su = stack(u.reshape(batch, channels, length), height, width, 1.0)
-    sdt = stack(dt.reshape(batch, channels, length), height, width, 1.0)
-    sb = stack(B.reshape(batch, groups * states, length), height, width, 1.0)
-    sc = stack(C.reshape(batch, groups * states, length), height, width, 1.0)
+    su, sdt, sb, sc = _stack_all(
+        [u.reshape(batch, channels, length), dt.reshape(batch, channels, length),
+         B.reshape(batch, groups * states, length), C.reshape(batch, groups * states, length)], height, width, 1.0)
     shape = (batch, 4 * groups, states, length)
     return su, sdt, A.repeat(4, 1).contiguous(), sb.view(shape), sc.view(shape)
 
@@ -175,12 +182,10 @@ class _PathScan(torch.autograd.Function):
         length = height * width
         sdy = _stack_impl(dy.to(ctx.u_dtype).contiguous().reshape(batch, channels, length), height, width, ctx.scale)
         dus, ddts, das, dbs, dcs, _, _, _ = selscan_bwd_impl(sdy, su, sdt, sa, sb, sc, None, None, None, False, ck)
-        merge = _merge_impl
-        du = merge(dus, height, width, 1.0).view(batch, channels, height, width)
-        ddt = merge(ddts, height, width, 1.0).view(batch, channels, height, width)
         rows = (batch, 4 * groups * states, length)
-        dB = merge(dbs.reshape(rows), height, width, 1.0).view(batch, groups, states, height, width)
-        dC = merge(dcs.reshape(rows), height, width, 1.0).view(batch, groups, states, height, width)
+        du, ddt, dB, dC = _merge_all([dus, ddts, dbs.reshape(rows), dcs.reshape(rows)], height, width, 1.0)
+        du, ddt = (t.view(batch, channels, height, width) for t in (du, ddt))
+        dB, dC = (t.view(batch, groups, states, height, width) for t in (dB, dC))
         dA = das.view(4, channels, states).sum(0)
         return du, ddt, dA, dB, dC, None
 
