@@ -952,6 +952,10 @@ fwd_lane(Geo g, Ptrs p) {
 //     silu(z) is exactly zero somewhere;
 //   - the workgroup's 4 wavefronts add their dB/dC blocks in a fixed order and write one
 //     partial per 16 channels (per 4 channels when a group is not a multiple of 16 wide).
+// It is bound by vector issue.  B and C pass through the transpose buffer, so a workgroup's LDS
+// (33.8 KB, 44 KB with a buffer of their own) and 128 registers allow four wavefronts a SIMD, and
+// A multiplies the second sum after the transpose, folded into its additions: at 4 x 5120 x 4096
+// 1154 -> 1107 us a launch.
 // A block's inputs are requested one block ahead.  Needs dstate <= 16, channels per group a
 // multiple of 4 and fp32 delta.  VBC: whole 16-step blocks, and 16-byte aligned rows of B and C.
 // Without it the last block's steps past the end take zeros for every input (what the loads
@@ -1067,12 +1071,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
 }
 
 template <class TU, class TB, bool VBC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VBC ? 4 : 3)))
 bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
   // per wavefront: the transposes of the pairs (h B, a x h); in blocks that need it, the
   // first terms first transpose C x; the workgroup's dB/dC blocks reuse the buffers
   __shared__ __align__(16) float lds[4][kTrFloats];
-  __shared__ __align__(16) float sbc[4][2][HS][kBcRow];  // B and C of the block (kBcRow)
   const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63, cl = lane >> 4, n = lane & 15;
   const int64_t first = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels;
@@ -1102,9 +1105,11 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
   const auto rB = raw_buffer(static_cast<const TB*>(p.B) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
   const auto rC = raw_buffer(static_cast<const TB*>(p.C) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
   const uint32_t eoff = static_cast<uint32_t>(cl) * L + n;
-  const auto share = BcShare<TB, VBC>::at(lane, N, L, &sbc[wave][0][0][0]);
-  const float* brow = &sbc[wave][0][n][0];
-  const float* crow = &sbc[wave][1][n][0];
+  // the block's B and C rows (kBcRow) pass through the same buffer: every lane has read its
+  // rows before the wavefront's first transpose write
+  const auto share = BcShare<TB, VBC>::at(lane, N, L, tr);
+  const float* brow = tr + n * kBcRow;
+  const float* crow = brow + HS * kBcRow;
   const int tw = cl * HS + n;  // this lane's column in a transpose row
   const int64_t sstep = g.dim * N;
   const float* sbase = p.states + ck_index(g, row0, 0, 0);
@@ -1184,6 +1189,7 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
     float bv[HS], cv[HS];
     lds_row<HS>(brow, bv);
     lds_row<HS>(crow, cv);
+    wave_lds_sync();
     // ---- recompute the block's states from the saved one
     float xh[HS], ah[HS];
     auto recompute = [&](auto with_y) {
@@ -1248,11 +1254,16 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
       float v[2 * HS];
       lds_row<2 * HS>(tr + n * kTrPitch + 2 * cl * HS, v);
       // the second sum's factor A of state m comes from lane m of the row: one rounding a term
-      float a[4] = {}, b[4] = {};
+      float a[4], b[4];
       static_for<0, HS>([&](auto mc) {
         constexpr int m = decltype(mc)::value;
-        a[m & 3] += v[2 * m];
-        b[m & 3] = fmaf(row_bcast<m>(an), v[2 * m + 1], b[m & 3]);
+        if constexpr (m < 4) {
+          a[m] = v[2 * m];
+          b[m] = row_bcast<m>(an) * v[2 * m + 1];
+        } else {
+          a[m & 3] += v[2 * m];
+          b[m & 3] = fmac_row<m>(b[m & 3], an, v[2 * m + 1]);
+        }
       });
       s1 = (a[0] + a[1]) + (a[2] + a[3]);
       s2 = (b[0] + b[1]) + (b[2] + b[3]);
