@@ -53,7 +53,8 @@ __global__ void __launch_bounds__(256) prep(Geo g, Ptrs p) {
 template <typename TM, bool VEC>
 __global__ void __launch_bounds__(256) cb_kernel(Geo g, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][2 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][2 * TE];
   // lower-triangular tile (i, j), j <= i
   const WgId id = wg_id(g.qb * (g.qb + 1) / 2, g.nc * g.ngroups);
   const int idx = id.x;
@@ -77,15 +78,20 @@ __global__ void __launch_bounds__(256) cb_kernel(Geo g, Ptrs p) {
     load_bw<TM, VEC>(g, Bm, b, tc + 64 * j, gg, 64 * k, r.b);
   };
   auto put = [&](int k, Regs& r) {
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     put_raw<TM, false>(buf, r0, c0, r.c[0], r.c[1]);       // A[l][n] = C_l[n]
     put_raw<TM, false>(buf + TE, r0, c0, r.b[0], r.b[1]);  // Bt[s][n] = B_s[n]
   };
   f32x16 acc;
   zero(acc);
-  Regs ra, rb;
-  pipeline2(g.nnt, ra, rb, fetch, put,
-            [&](int k) { mma_tile<TM>(acc, sbuf[k & 1], sbuf[k & 1] + TE, wm, wn, lane, 64); });
+  auto mma = [&](int k) { mma_tile<TM>(acc, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64); };
+  Regs ra;
+  if constexpr (NB == 1) {
+    pipeline1(g.nnt, ra, fetch, put, mma);
+  } else {
+    Regs rb;
+    pipeline2(g.nnt, ra, rb, fetch, put, mma);
+  }
   TM* out = static_cast<TM*>(p.cb) + ((b * g.nc + c) * g.ngroups + gg) * g.q * g.q;
 #pragma unroll
   for (int r = 0; r < 16; ++r)
@@ -126,9 +132,10 @@ __global__ void __launch_bounds__(256) state_pass(Geo g, Ptrs p) {
 }
 
 template <typename TM, bool VEC>
-__global__ void __launch_bounds__(256) chunk_scan(Geo g, Ptrs p) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TM) == 2 ? 2 : 3)))
+chunk_scan(Geo g, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][2 * TE];
+  __shared__ __align__(16) TM sbuf[kStageBufs<TM>][2 * TE];
   __shared__ __align__(16) float csc[256], dlc[256], ecol[256], dcol[64];
   // Heads fastest: the workgroups that run together share the group's C and C B^T
   // tiles and cover whole token rows of x and the outputs.
@@ -591,9 +598,7 @@ static void launch_fwd_t(const Geo& g, const Ptrs& q, hipStream_t s) {
   MKO_TIMED("ssd_prep", s, prep<<<dim3(g.nc, g.nheads, g.batch), 256, 0, s>>>(g, q));
   MKO_TIMED("ssd_cb", s,
             cb_kernel<TM, VEC><<<dim3(g.qb * (g.qb + 1) / 2 * g.nc * g.ngroups * g.batch), 256, 0, s>>>(g, q));
-  const dim3 cs_grid(g.npt * g.nnp * g.nc * bh);
-  if (g.qb == 4) MKO_TIMED("ssd_chunk_state", s, chunk_state<TM, VEC, false, 4><<<cs_grid, 256, 0, s>>>(g, q, q.states));
-  else MKO_TIMED("ssd_chunk_state", s, chunk_state<TM, VEC, false><<<cs_grid, 256, 0, s>>>(g, q, q.states));
+  launch_chunk_state<TM, VEC, false>(g, q, q.states, s);
   MKO_TIMED("ssd_state_pass", s,
             state_pass<TM><<<dim3(static_cast<unsigned>((g.headdim * g.dstate + 2047) / 2048), bh), 256, 0, s>>>(
                 g, q));

@@ -183,13 +183,15 @@ __device__ __forceinline__ void scale8(const V8<TM>& v, float s, float (&f)[8]) 
 // are staged transposed.  Double-buffered: the loads of the next 64 tokens are in
 // flight during the products of the current ones.
 // QB > 0: the chunk has QB 64-token tiles (a compile-time stage count, with the loads of
-// up to three stages in flight); QB = 0: qb at run time, two stages in flight.
+// up to three stages in flight); QB = 0: qb at run time, two stages in flight (fp32: one, on a
+// single buffer, see kStageBufs; 4 x 1024 tokens, 32 heads, d_state 128: 57 -> 43 us)
 template <typename TM, bool VEC, bool BWD, int QB = 0>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TM) == 2 ? 3 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 chunk_state(Geo g, Ptrs p, void* out_) {
   constexpr int LD = compact_ld<TM>();  // LDS bounds this kernel: the compact tiles
   constexpr int TE = LdsTile<TM, LD>::elems;
-  __shared__ __align__(16) TM sbuf[2][3 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][3 * TE];
   __shared__ float s1[256];
   const WgId id = wg_id(g.npt * g.nnp, g.nc);
   const int pt = id.x / g.nnp, np = id.x % g.nnp;
@@ -220,7 +222,7 @@ chunk_state(Geo g, Ptrs p, void* out_) {
   };
   auto put = [&](auto kc, Regs& r) {
     const int kb = kc;
-    TM* buf = sbuf[kb & 1];
+    TM* buf = sbuf[kb % NB];
     float a[8], bb[8];
     scale8(r.x[0], s1[64 * kb + r0], a);
     scale8(r.x[1], s1[64 * kb + r0 + 1], bb);
@@ -233,14 +235,18 @@ chunk_state(Geo g, Ptrs p, void* out_) {
   zero(acc1);
   __syncthreads();  // s1
   auto mma = [&](auto kc) {
-    TM* buf = sbuf[static_cast<int>(kc) & 1];
+    TM* buf = sbuf[static_cast<int>(kc) % NB];
     mma_tile<TM, LD>(acc0, buf, buf + TE, wm, wn, lane, 64);
     mma_tile<TM, LD>(acc1, buf, buf + 2 * TE, wm, wn, lane, 64);
   };
+  static_assert(QB == 0 || NB == 2, "a compile-time stage count takes two buffers");
   if constexpr (QB > 0) {
     constexpr int D = QB < 3 ? QB : 3;
     Regs regs[D];
     pipeline_static<QB, D>(regs, fetch, put, mma);
+  } else if constexpr (NB == 1) {
+    Regs r;
+    pipeline1(g.qb, r, fetch, put, mma);
   } else {
     Regs ra, rb;
     pipeline2(g.qb, ra, rb, fetch, put, mma);
@@ -259,6 +265,19 @@ chunk_state(Geo g, Ptrs p, void* out_) {
     store_win<TM, VEC>(out + 64 * kk, static_cast<int>(g.dstate), clamp64(g.headdim - pc0),
                        static_cast<int>(g.dstate - nn0 - 64 * kk), v[0], v[1]);
   }
+}
+
+template <typename TM, bool VEC, bool BWD>
+inline void launch_chunk_state(const Geo& g, const Ptrs& q, void* out, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(g.npt * g.nnp * g.nc * g.batch * g.nheads));
+  const char* name = BWD ? "ssd_chunk_state_bwd" : "ssd_chunk_state";
+  if constexpr (sizeof(TM) == 2) {
+    if (g.qb == 4) {
+      MKO_TIMED(name, s, chunk_state<TM, VEC, BWD, 4><<<grid, 256, 0, s>>>(g, q, out));
+      return;
+    }
+  }
+  MKO_TIMED(name, s, chunk_state<TM, VEC, BWD><<<grid, 256, 0, s>>>(g, q, out));
 }
 
 // Loads cs and step of a whole chunk into LDS (q <= 256 values each), and the column
@@ -366,8 +385,9 @@ __device__ __forceinline__ void chunk_out(const Geo& g, const Ptrs& p, f32x16& a
       load_xw<TM, VEC>(g, X, b, tc + 64 * j, h, pc0, r.b);                      // x rows s
     }
   };
+  constexpr int NB = kStageBufs<TM>;
   auto put = [&](int k, Regs& r) {
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     float a[8], bb[8];
     if (k < g.nnt) {
       scale8(r.a[0], e0, a);
@@ -384,8 +404,18 @@ __device__ __forceinline__ void chunk_out(const Geo& g, const Ptrs& p, f32x16& a
     }
   };
   zero(acc);
-  Regs ra, rb;
-  auto mma = [&](int k) { mma_tile<TM>(acc, sbuf[k & 1], sbuf[k & 1] + TE, wm, wn, lane, 64); };
+  Regs ra;
+  auto mma = [&](int k) { mma_tile<TM>(acc, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64); };
+  if constexpr (NB == 1) {
+    if constexpr (EPI) {
+      pipeline1e(n, ra, fetch, put, mma, [&](const Regs& r) { epi(r.a, r.b); });
+    } else {
+      pipeline1(n, ra, fetch, put, mma);
+      __syncthreads();
+    }
+    return;
+  }
+  Regs rb;
   if constexpr (EPI) {
     pipeline2e(n, ra, rb, fetch, put, mma, [&](const Regs& r) {
       __syncthreads();

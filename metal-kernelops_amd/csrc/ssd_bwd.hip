@@ -116,7 +116,7 @@ __device__ __forceinline__ void dd_columns(float (&dd)[8], float* colred, float*
 template <typename TM, bool VEC, bool SAVED>
 __global__ void __launch_bounds__(256) gate(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][2 * TE];
+  __shared__ __align__(16) TM sbuf[kStageBufs<TM>][2 * TE];
   __shared__ __align__(16) float csc[256], dlc[256], ecol[256];
   __shared__ float colred[4][64];
   // Heads fastest: the workgroups that run together cover whole token rows (a row's
@@ -403,7 +403,8 @@ __global__ void __launch_bounds__(256) state_rev(Geo g, BwdPlan pl, Ptrs p) {
 template <typename TM, bool VEC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) du_kernel(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][2 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][2 * TE];
   __shared__ __align__(16) float csc[256], dlc[256], ecol[256], dcol[64];
   const int nj = (g.qb + 1) / 2;
   // heads fastest, as in the forward's chunk_scan
@@ -474,7 +475,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) d
   auto put = [&](int k, Regs& r) {
     int j, kk;
     tile_of(k, j, kk);
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     float a[8], bb[8];
     if (kk < g.nnt) {
       const float w0 = fast_exp(T - csc[64 * j + r0]), w1 = fast_exp(T - csc[64 * j + r0 + 1]);
@@ -543,20 +544,28 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) d
     if (j != jb) load_xw<TM, VEC>(g, static_cast<const TM*>(p.x), b, tc + 64 * jb, h, pc0, xv);
     __syncthreads();  // red is refilled by the next stage
   };
-  Regs ra, rb;
-  pipeline2(n, ra, rb, fetch, put, [&](int k) {
-    mma_tile<TM>(acc, sbuf[k & 1], sbuf[k & 1] + TE, wm, wn, lane, 64);
+  auto mma = [&](int k) {
+    mma_tile<TM>(acc, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64);
     int j, kk;
     tile_of(k, j, kk);
-    // buffer (k+1)&1 was last read by stage k-1, which every wave finished before the
+    // with two buffers, (k+1)&1 was last read by stage k-1, which every wave finished before the
     // barrier that published stage k
-    float* red = reinterpret_cast<float*>(&sbuf[(k + 1) & 1][0]);
-    if (kk == g.nnt - 1) tau_snapshot(j, red);
-    if (kk == g.nnt + g.qb - j - 1) {
+    float* red = reinterpret_cast<float*>(&sbuf[(k + 1) % NB][0]);
+    const bool snap = kk == g.nnt - 1, last = kk == g.nnt + g.qb - j - 1;
+    if (NB == 1 && (snap || last)) __syncthreads();
+    if (snap) tau_snapshot(j, red);
+    if (last) {
       epilogue(j, red);
       zero(acc);
     }
-  });
+  };
+  Regs ra;
+  if constexpr (NB == 1) {
+    pipeline1(n, ra, fetch, put, mma);
+  } else {
+    Regs rb;
+    pipeline2(n, ra, rb, fetch, put, mma);
+  }
 }
 
 // Stage k of du_mt's schedule: s-tile j, then its state stages kk < nnt and its intra
@@ -930,9 +939,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) d
 // Adjoint of C.B^T for one lower tile (i, j) of a chunk, summed over a block of the
 // group's heads: sum_h (gy_i u_j^T) o e^{cs_l - cs_s}.
 template <typename TM, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) dcb_kernel(Geo g, BwdPlan pl, Ptrs p) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TM) == 2 ? 4 : 3)))
+dcb_kernel(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][2 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][2 * TE];
   __shared__ float csr[2][64], css[2][64];
   const WgId id = wg_id(pl.npairs * pl.hb1, g.nc * g.ngroups);
   const int pair = id.x / pl.hb1, hb = id.x % pl.hb1;
@@ -969,7 +980,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
   };
   auto put = [&](int k, Regs& r) {
     const int hh = k / g.npt, pt = k % g.npt;
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     float a[8], bb[8];
     put_raw<TM, false>(buf, r0, c0, r.gm[0], r.gm[1]);  // A[l][p] = gy_l[p]
     scale8(r.xm[0], r.dls[0], a);
@@ -986,10 +997,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
     // diagonal tile: per head, the product times e^{cs_l - cs_s} below the diagonal
     f32x16 w;
     zero(w);
-    Regs ra, rb;
-    pipeline2(nst, ra, rb, fetch, put, [&](int k) {
+    auto mma = [&](int k) {
       const int hh = k / g.npt, pt = k % g.npt;
-      mma_tile<TM>(w, sbuf[k & 1], sbuf[k & 1] + TE, wm, wn, lane, 64);
+      mma_tile<TM>(w, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64);
       if (pt == g.npt - 1) {
         const float cs_s = css[hh & 1][acc_col(wn, lane)];
 #pragma unroll
@@ -999,7 +1009,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
         }
         zero(w);
       }
-    });
+    };
+    Regs ra;
+    if constexpr (NB == 1) {
+      pipeline1(nst, ra, fetch, put, mma);
+    } else {
+      Regs rb;
+      pipeline2(nst, ra, rb, fetch, put, mma);
+    }
   } else {
     // i > j: e^{cs_l - cs_s} = e^{cs_l - cs_e} e^{cs_e - cs_s} (e = the last token of
     // tile j, both factors at most 1 for a non-increasing cs) goes into the operands'
@@ -1023,7 +1040,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
       r.ce = p.cs[so + 64 * j + 63];
     };
     auto put_o = [&](int k, RegsO& r) {
-      TM* buf = sbuf[k & 1];
+      TM* buf = sbuf[k % NB];
       float a[8], bb[8];
       scale8(r.gm[0], fast_exp(r.ci[0] - r.ce), a);
       scale8(r.gm[1], fast_exp(r.ci[1] - r.ce), bb);
@@ -1032,9 +1049,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
       scale8(r.xm[1], r.dls[1] * fast_exp(r.ce - r.cj[1]), bb);
       put2x8<TM, false>(buf + TE, r0, c0, a, bb);  // Bt[s][p] = e^{cs_e - cs_s} step_s x_s[p]
     };
-    RegsO ra, rb;
-    pipeline2(nst, ra, rb, fetch_o, put_o,
-              [&](int k) { mma_tile<TM>(dacc, sbuf[k & 1], sbuf[k & 1] + TE, wm, wn, lane, 64); });
+    auto mma = [&](int k) { mma_tile<TM>(dacc, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64); };
+    RegsO ra;
+    if constexpr (NB == 1) {
+      pipeline1(nst, ra, fetch_o, put_o, mma);
+    } else {
+      RegsO rb;
+      pipeline2(nst, ra, rb, fetch_o, put_o, mma);
+    }
   }
   float* out = p.dcb + (((b * g.nc + c) * g.ngroups + gg) * pl.hb1 + hb) * g.q * g.q;
 #pragma unroll
@@ -1046,11 +1068,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) d
 // sum_h e^{cs_l} gy_l S_in) for one 64-token tile and two d_state tiles, over a
 // block of the group's heads.
 template <typename TM, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TM) == 2 ? 3 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 dbc_state(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int LD = compact_ld<TM>();  // LDS bounds this kernel: the compact tiles
   constexpr int TE = LdsTile<TM, LD>::elems;
-  __shared__ __align__(16) TM sbuf[2][3 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][3 * TE];
   const WgId id = wg_id(g.qb * g.nnp * 2 * pl.hb2, g.nc * g.ngroups);
   int idx = id.x;
   const int hb = idx % pl.hb2;
@@ -1093,7 +1116,7 @@ dbc_state(Geo g, BwdPlan pl, Ptrs p) {
     r.T = p.cs[so + g.q - 1];
   };
   auto put = [&](int k, Regs& r) {
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     float a[8], bb[8];
     const float sc0 = which ? fast_exp(r.cl[0]) : r.dl[0] * fast_exp(r.T - r.cl[0]);
     const float sc1 = which ? fast_exp(r.cl[1]) : r.dl[1] * fast_exp(r.T - r.cl[1]);
@@ -1106,12 +1129,18 @@ dbc_state(Geo g, BwdPlan pl, Ptrs p) {
   f32x16 acc0, acc1;
   zero(acc0);
   zero(acc1);
-  Regs ra, rb;
-  pipeline2(nst, ra, rb, fetch, put, [&](int k) {
-    TM* buf = sbuf[k & 1];
+  auto mma = [&](int k) {
+    TM* buf = sbuf[k % NB];
     mma_tile<TM, LD>(acc0, buf, buf + TE, wm, wn, lane, 64);
     mma_tile<TM, LD>(acc1, buf, buf + 2 * TE, wm, wn, lane, 64);
-  });
+  };
+  Regs ra;
+  if constexpr (NB == 1) {
+    pipeline1(nst, ra, fetch, put, mma);
+  } else {
+    Regs rb;
+    pipeline2(nst, ra, rb, fetch, put, mma);
+  }
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int64_t t = tl0 + acc_row(wm, lane, r);
@@ -1128,7 +1157,8 @@ dbc_state(Geo g, BwdPlan pl, Ptrs p) {
 template <typename TM, bool VEC>
 __global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
-  __shared__ __align__(16) TM sbuf[2][3 * TE];
+  constexpr int NB = kStageBufs<TM>;
+  __shared__ __align__(16) TM sbuf[NB][3 * TE];
   const WgId id = wg_id(g.qb * g.nnp * 2, g.nc * g.ngroups);
   int idx = id.x;
   const int which = idx % 2;
@@ -1169,7 +1199,7 @@ __global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
     load_bw<TM, VEC>(g, Om, b, ot0, gg, nn0 + 64, r.o1);
   };
   auto put = [&](int k, Regs& r) {
-    TM* buf = sbuf[k & 1];
+    TM* buf = sbuf[k % NB];
     if (which)
       put2x8<TM, false>(buf, r0, c0, r.kf[0], r.kf[1]);  // A[l][s] = dCB[l][s]
     else
@@ -1180,12 +1210,18 @@ __global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
   f32x16 acc0, acc1;
   zero(acc0);
   zero(acc1);
-  Regs ra, rb;
-  pipeline2(nst, ra, rb, fetch, put, [&](int k) {
-    TM* buf = sbuf[k & 1];
+  auto mma = [&](int k) {
+    TM* buf = sbuf[k % NB];
     mma_tile<TM>(acc0, buf, buf + TE, wm, wn, lane, 64);
     mma_tile<TM>(acc1, buf, buf + 2 * TE, wm, wn, lane, 64);
-  });
+  };
+  Regs ra;
+  if constexpr (NB == 1) {
+    pipeline1(nst, ra, fetch, put, mma);
+  } else {
+    Regs rb;
+    pipeline2(nst, ra, rb, fetch, put, mma);
+  }
   __syncthreads();
   float* red = reinterpret_cast<float*>(&sbuf[0][0]);
   TM* out = static_cast<TM*>(which ? p.dC : p.dB);
@@ -1498,11 +1534,7 @@ int launch_bwd_t(const Geo& g, const BwdPlan& pl, const Ptrs& q, hipStream_t s) 
       MKO_TIMED("ssd_gate", s, gate<TM, VEC, true><<<dim3(g.qb * g.npt * g.nc * bh), 256, 0, s>>>(g, pl, q));
     else
       MKO_TIMED("ssd_gate", s, gate<TM, VEC, false><<<dim3(g.qb * g.npt * g.nc * bh), 256, 0, s>>>(g, pl, q));
-    const dim3 cs_grid(g.npt * g.nnp * g.nc * bh);
-    if (g.qb == 4)
-      MKO_TIMED("ssd_chunk_state_bwd", s, chunk_state<TM, VEC, true, 4><<<cs_grid, 256, 0, s>>>(g, q, q.dstates));
-    else
-      MKO_TIMED("ssd_chunk_state_bwd", s, chunk_state<TM, VEC, true><<<cs_grid, 256, 0, s>>>(g, q, q.dstates));
+    launch_chunk_state<TM, VEC, true>(g, q, q.dstates, s);
   }
   auto dcb = [&](hipStream_t st) {
     MKO_TIMED("ssd_dcb", st, dcb_kernel<TM, VEC><<<dim3(pl.npairs * pl.hb1 * ncg * nb), 256, 0, st>>>(g, pl, q));

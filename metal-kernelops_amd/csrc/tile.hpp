@@ -235,6 +235,40 @@ __device__ __forceinline__ void pipeline2(int n, Regs& ra, Regs& rb, Fetch&& fet
   }
 }
 
+// Operand buffers of a staged product.  Two let one barrier a stage do, but two of fp32 (16.5 KB
+// a 64x64 tile) leave a kernel one or two workgroups per CU, too few to hide what a stage waits
+// for: fp32 takes one buffer, two barriers a stage, and three or four workgroups.
+template <typename TM>
+constexpr int kStageBufs = sizeof(TM) == 2 ? 2 : 1;
+
+// pipeline2 on a single operand buffer: the next stage's loads fly during the products.
+template <class Regs, class Fetch, class Put, class Mma>
+__device__ __forceinline__ void pipeline1(int n, Regs& r, Fetch&& fetch, Put&& put, Mma&& mma) {
+  fetch(0, r);
+  for (int k = 0; k < n; ++k) {
+    put(k, r);
+    __syncthreads();
+    if (k + 1 < n) fetch(k + 1, r);
+    mma(k);
+    if (k + 1 < n) __syncthreads();
+  }
+}
+
+// pipeline1 whose fetch past the last stage, n, loads the epilogue's inputs; epi(regs) runs once
+// every wave is done with the buffer.
+template <class Regs, class Fetch, class Put, class Mma, class Epi>
+__device__ __forceinline__ void pipeline1e(int n, Regs& r, Fetch&& fetch, Put&& put, Mma&& mma, Epi&& epi) {
+  fetch(0, r);
+  for (int k = 0; k < n; ++k) {
+    put(k, r);
+    __syncthreads();
+    fetch(k + 1, r);
+    mma(k);
+    __syncthreads();
+  }
+  epi(r);
+}
+
 // f(Int<K>{}) for K = B .. E-1, each call with K a compile-time constant.
 template <int K>
 struct Int {
