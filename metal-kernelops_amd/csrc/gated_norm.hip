@@ -21,6 +21,8 @@
 // Groups wider than the register set stream: the forward walks the group twice (sum
 // of squares, then the write); the backward computes c1 per (row, group) in one kernel
 // and dx/dz and the dw/db partials with one thread per vector column in another.
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace mko {
@@ -32,8 +34,8 @@ constexpr int kStream = 1024;       // threads of the streaming kernels' team
 constexpr int kFwdElems = 32;       // register elements per thread, forward
 constexpr int kBwdElems = 8;        // register elements per thread, backward
 constexpr int kBwdTeamWaves = 8;    // waves per backward workgroup when teams are narrow
-constexpr int kBwdWaveTarget = 8192;  // backward waves across the chip without parameter gradients
-constexpr int kBwdWaveTargetParams = 4096;  // ... with them (each row block adds a partial row)
+constexpr int kCus = 256;
+constexpr int kBwdCuWaves = 20;     // backward waves a CU holds
 constexpr int kMaxBlocks = 4096;      // row blocks per group: two column-sum passes of 64 rows
 constexpr int kColThreads = 256;    // workgroup of the per-column backward kernel
 
@@ -791,8 +793,12 @@ Plan make_plan(const mko_gated_norm_params* p, bool bwd) {
   if (bwd) {
     if (pl.path == kDense) {
       const int64_t wg_waves = static_cast<int64_t>(g.tpw) * (g.tw / kWave);
-      const int64_t target = g.want_dw || g.want_db ? kBwdWaveTargetParams : kBwdWaveTarget;
-      int64_t blocks = cdiv(cdiv(target, wg_waves), g.ngroups);
+      // As many workgroups as the chip holds at once (256 CUs, five wavefronts on each of their
+      // four SIMDs), or twice that without partial rows, whose sums grow with them: with a
+      // wavefront count alone (4096: 410 workgroups of ten at 5120 features) some CUs had two and
+      // some one for the whole kernel (8192 x 5120 bf16, gate before, dweight: 104 -> 89 us).
+      const int64_t held = kCus * std::max<int64_t>(1, kBwdCuWaves / wg_waves);
+      int64_t blocks = (g.want_dw || g.want_db ? held : 2 * held) / g.ngroups;
       blocks = blocks > kMaxBlocks ? kMaxBlocks : blocks;
       const int64_t most = cdiv(g.rows, g.tpw);
       blocks = blocks > most ? most : blocks;
