@@ -290,3 +290,24 @@ def test_decode_steps_equal_prefill():
     outs = [causal_conv1d_update(x[..., t], state, w, b, "silu") for t in range(12)]
     assert rel(torch.stack(outs, dim=-1), want) <= 1e-6
     assert torch.equal(state, final)
+
+
+# Rows of one block and less, one and two wavefront iterations (512 steps each) with a whole and a
+# ragged end, and both sides of a wavefront's 4096 steps, where the gradients cross to the next one.
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("length", [1, 7, 8, 511, 512, 513, 520, 1027, 4095, 4096, 4099, 4104])
+@pytest.mark.parametrize("width", [2, 4, 7])
+def test_backward_walk_edges(width, length, dtype):
+    from metal_kernelops.cv import causal_conv1d_fn
+    b, c = 2, 3
+    x, w, bias = make((b, c, length), 1, dtype=dtype), make((c, width), 2, dtype=dtype), make((c,), 3, dtype=dtype)
+    init, dy = make((b, c, width - 1), 4, dtype=dtype), make((b, c, length), 5, dtype=dtype)
+    got = [t.to(DEV).requires_grad_(True) for t in (x, w, bias, init)]
+    out = causal_conv1d_fn(got[0], got[1], got[2], "silu", got[3])
+    grads = torch.autograd.grad(out, got, dy.to(DEV))
+    ref = [t.double().requires_grad_(True) for t in (x, w, bias, init)]
+    want = torch.autograd.grad(oracle.causal_conv1d(ref[0], ref[1], ref[2], "silu", ref[3])[0], ref, dy.double())
+    tol = 1e-4 if dtype == torch.float32 else 2e-2
+    for name, g, r in zip(("x", "weight", "bias", "initial"), grads, want):
+        assert rel(g, r) <= tol, (name, rel(g, r))
