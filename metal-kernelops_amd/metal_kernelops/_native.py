@@ -262,6 +262,25 @@ def code(dtype):
     return _DTYPE_CODE[dtype]
 
 
+def plain_call(*tensors):
+    """Whether a call on ``tensors`` (None among them allowed) is an ordinary eager one that no
+    gradient, tracer or mode has to see, so that the implementation behind a custom op may be
+    called without the dispatcher: its round trip costs 10-25 us of host time, as much as the
+    kernels of a short prompt.  Not plain: grad mode with an input that requires grad, compiling
+    or tracing, tensor subclasses, dispatch or function modes, functorch transforms and
+    forward-mode levels; those go through the op, which does with them what it always did."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() \
+            or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None \
+            or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
+                              or (grad and t.requires_grad)):
+            return False
+    return True
+
+
 def stream_of(device):
     return torch.cuda.current_stream(device).cuda_stream
 

@@ -100,8 +100,7 @@ def _params(x, weight, bias, init, silu):
     return p
 
 
-@torch.library.custom_op("mko::conv1d_fwd", mutates_args=(), device_types="cuda")
-def _conv1d_fwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Optional[Tensor], silu: bool,
+def _conv1d_fwd_impl(x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Optional[Tensor], silu: bool,
                 write_final: bool) -> Tuple[Tensor, Tensor]:
     out = torch.empty_like(x)
     final = x.new_empty(x.shape[0], x.shape[1], weight.shape[1] - 1 if write_final else 0)
@@ -114,13 +113,15 @@ def _conv1d_fwd(x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Optiona
     return out, final
 
 
+_conv1d_fwd = torch.library.custom_op("mko::conv1d_fwd", _conv1d_fwd_impl, mutates_args=(), device_types="cuda")
+
+
 @_conv1d_fwd.register_fake
 def _(x, weight, bias, init, silu, write_final):
     return torch.empty_like(x), x.new_empty(x.shape[0], x.shape[1], weight.shape[1] - 1 if write_final else 0)
 
 
-@torch.library.custom_op("mko::conv1d_bwd", mutates_args=(), device_types="cuda")
-def _conv1d_bwd(dout: Tensor, x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Optional[Tensor],
+def _conv1d_bwd_impl(dout: Tensor, x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Optional[Tensor],
                 silu: bool, need_weight: bool, need_bias: bool, need_init: bool
                 ) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     channels, width = weight.shape
@@ -145,6 +146,9 @@ def _conv1d_bwd(dout: Tensor, x: Tensor, weight: Tensor, bias: Optional[Tensor],
     return dx, dweight, dbias, dinit
 
 
+_conv1d_bwd = torch.library.custom_op("mko::conv1d_bwd", _conv1d_bwd_impl, mutates_args=(), device_types="cuda")
+
+
 @_conv1d_bwd.register_fake
 def _(dout, x, weight, bias, init, silu, need_weight, need_bias, need_init):
     channels, width = weight.shape
@@ -162,7 +166,10 @@ def _setup(ctx, inputs, output):
 def _backward(ctx, dout, _dfinal):
     x, weight, bias, init = ctx.saved_tensors
     need = ctx.needs_input_grad
-    dx, dweight, dbias, dinit = torch.ops.mko.conv1d_bwd(
+    backward = torch.ops.mko.conv1d_bwd
+    if not torch.is_grad_enabled() and nat.plain_call(dout, x, weight, bias, init):
+        backward = _conv1d_bwd_impl
+    dx, dweight, dbias, dinit = backward(
         dout.contiguous(), x, weight, bias, init, ctx.silu, bool(need[1]), bool(need[2] and bias is not None),
         bool(need[3] and init is not None))
     return (dx, dweight if need[1] else None, dbias if need[2] and bias is not None else None,
@@ -268,8 +275,9 @@ def causal_conv1d_fn(x, weight, bias=None, activation=None, initial_state=None, 
     # without autograd the kernel writes the final state; with it, the final state is a
     # slice of cat(initial_state, x) so that its gradient reaches both
     fused_final = return_final_state and not grads
-    out, final = torch.ops.mko.conv1d_fwd(work, weight.contiguous(), shift, init, activation is not None,
-                                          bool(fused_final and work.numel()))
+    args = (work, weight.contiguous(), shift, init)
+    forward = _conv1d_fwd_impl if nat.plain_call(*args) else torch.ops.mko.conv1d_fwd
+    out, final = forward(*args, activation is not None, bool(fused_final and work.numel()))
     out = out.to(x.dtype)
     if not return_final_state:
         return out

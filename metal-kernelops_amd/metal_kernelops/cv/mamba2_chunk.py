@@ -114,8 +114,7 @@ def _params(x, dt, A, B, C, D, z, dt_bias, init, softplus, save_y=False):
     return p
 
 
-@torch.library.custom_op("mko::ssd_fwd", mutates_args=(), device_types="cuda")
-def _ssd_fwd(x: Tensor, dt: Tensor, A: Tensor, B: Tensor, C: Tensor, D: Optional[Tensor],
+def _ssd_fwd_impl(x: Tensor, dt: Tensor, A: Tensor, B: Tensor, C: Tensor, D: Optional[Tensor],
              z: Optional[Tensor], dt_bias: Optional[Tensor], initial_states: Optional[Tensor],
              softplus: bool, save_y: bool) -> Tuple[Tensor, Tensor, Tensor]:
     batch, length, nheads, headdim = x.shape
@@ -129,6 +128,9 @@ def _ssd_fwd(x: Tensor, dt: Tensor, A: Tensor, B: Tensor, C: Tensor, D: Optional
     return y, final, saved
 
 
+_ssd_fwd = torch.library.custom_op("mko::ssd_fwd", _ssd_fwd_impl, mutates_args=(), device_types="cuda")
+
+
 @_ssd_fwd.register_fake
 def _(x, dt, A, B, C, D, z, dt_bias, initial_states, softplus, save_y):
     batch, length, nheads, headdim = x.shape
@@ -136,8 +138,7 @@ def _(x, dt, A, B, C, D, z, dt_bias, initial_states, softplus, save_y):
             x.new_empty(0, dtype=torch.uint8))
 
 
-@torch.library.custom_op("mko::ssd_bwd", mutates_args=(), device_types="cuda")
-def _ssd_bwd(dy: Tensor, dfinal: Optional[Tensor], x: Tensor, dt: Tensor, A: Tensor, B: Tensor,
+def _ssd_bwd_impl(dy: Tensor, dfinal: Optional[Tensor], x: Tensor, dt: Tensor, A: Tensor, B: Tensor,
              C: Tensor, D: Optional[Tensor], z: Optional[Tensor], dt_bias: Optional[Tensor],
              initial_states: Optional[Tensor], softplus: bool, save_y: bool, saved: Tensor
              ) -> Tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -164,6 +165,9 @@ def _ssd_bwd(dy: Tensor, dfinal: Optional[Tensor], x: Tensor, dt: Tensor, A: Ten
     return dx, ddt, dA, dB, dC, dD, dz, dbias, dinit
 
 
+_ssd_bwd = torch.library.custom_op("mko::ssd_bwd", _ssd_bwd_impl, mutates_args=(), device_types="cuda")
+
+
 @_ssd_bwd.register_fake
 def _(dy, dfinal, x, dt, A, B, C, D, z, dt_bias, initial_states, softplus, save_y, saved):
     def f(shape):
@@ -187,7 +191,10 @@ def _backward(ctx, dy, dfinal, _dsaved):
     x, dt, A, B, C, D, z, bias, init, saved = ctx.saved_tensors
     if dy is None:
         dy = torch.zeros_like(x)
-    dx, ddt, dA, dB, dC, dD, dz, dbias, dinit = torch.ops.mko.ssd_bwd(
+    backward = torch.ops.mko.ssd_bwd
+    if not torch.is_grad_enabled() and nat.plain_call(dy, dfinal, x, dt, A, B, C, D, z, bias, init, saved):
+        backward = _ssd_bwd_impl
+    dx, ddt, dA, dB, dC, dD, dz, dbias, dinit = backward(
         dy.contiguous(), None if dfinal is None else dfinal.contiguous(), x, dt, A, B, C, D, z, bias,
         init, ctx.softplus, ctx.save_y, saved)
     return (dx, ddt, dA, dB, dC, dD if D is not None else None, dz if z is not None else None,
@@ -255,8 +262,9 @@ def mamba2_chunk_scan(x, dt, A, B, C, chunk_size=64, D=None, z=None, dt_bias=Non
     # The forward keeps its chunk output for the backward only when a gradient will be taken.
     save_y = torch.is_grad_enabled() and any(
         t is not None and t.requires_grad for t in (x, dt, A, B, C, D, z, dt_bias, initial_states))
-    y, final, _ = torch.ops.mko.ssd_fwd(x, dt, A, B, C, D, z, dt_bias, initial_states,
-                                        bool(dt_softplus), bool(save_y))
+    args = (x, dt, A, B, C, D, z, dt_bias, initial_states)
+    forward = _ssd_fwd_impl if nat.plain_call(*args) else torch.ops.mko.ssd_fwd
+    y, final, _ = forward(*args, bool(dt_softplus), bool(save_y))
     return y, final
 
 

@@ -154,7 +154,10 @@ def _backward(ctx, dout, _dstates):
     if dout is None:
         return (None,) * 9
     u, delta, A, B, C, D, z, bias, states, out = ctx.saved_tensors
-    du, ddelta, dA, dB, dC, dD, dz, dbias = torch.ops.mko.selscan_bwd(
+    backward = torch.ops.mko.selscan_bwd
+    if not torch.is_grad_enabled() and nat.plain_call(dout, u, delta, A, B, C, D, z, bias, states, out):
+        backward = selscan_bwd_impl
+    du, ddelta, dA, dB, dC, dD, dz, dbias = backward(
         dout.contiguous(), u, delta, A, B, C, D, z, bias, ctx.softplus, states, out)
     return (du, ddelta, dA, dB, dC, dD if D is not None else None, dz if z is not None else None,
             dbias if bias is not None else None, None)
@@ -217,8 +220,9 @@ def _run(u, dt, A, B, C, D, z, delta_bias, softplus):
     A, D, delta_bias = (None if t is None else t.contiguous() for t in f32)
     u, dt, B, C = (t.contiguous() for t in (u, dt, B, C))
     z = None if z is None else z.contiguous()
-    out, _ = torch.ops.mko.selscan_fwd(u, dt, A, B, C, D, z, delta_bias, bool(softplus))
-    return out
+    args = (u, dt, A, B, C, D, z, delta_bias)
+    forward = selscan_fwd_impl if nat.plain_call(*args) else torch.ops.mko.selscan_fwd
+    return forward(*args, bool(softplus))[0]
 
 
 def scan_mps(u, dt, A, B, C):
