@@ -344,8 +344,7 @@ struct WgId {
   int64_t z;
 };
 constexpr int kXcds = 8;
-__device__ __forceinline__ WgId wg_id(int nx, int ny) {
-  const int64_t total = gridDim.x, w = blockIdx.x;
+__device__ __forceinline__ WgId wg_id(int nx, int ny, int64_t w, int64_t total) {
   const int64_t per = total / kXcds;
   const int64_t lid = (w < per * kXcds) ? (w % kXcds) * per + w / kXcds : w;
   WgId r;
@@ -355,6 +354,7 @@ __device__ __forceinline__ WgId wg_id(int nx, int ny) {
   r.z = rest / ny;
   return r;
 }
+__device__ __forceinline__ WgId wg_id(int nx, int ny) { return wg_id(nx, ny, blockIdx.x, gridDim.x); }
 
 // Error reporting for the C ABI (defined in abi.hip).
 void mko_set_error(const char* fmt, ...);

@@ -2,9 +2,9 @@
 //
 // The sequence is cut into chunks of q = 64*qb tokens; inside a chunk every
 // contraction is done on 64x64 tiles on the matrix cores (mma.hpp):
-//   prep        per (b, h, chunk): step = softplus(dt + bias), cs = cumsum(step * A)
-//   cb          per (b, chunk, group), lower tiles: CB = C . B^T      (shared by the heads)
-//   chunk_state per (b, h, chunk): S = sum_l step_l e^{T - cs_l} x_l (x) B_l   (P x N)
+//   chunk_state per (b, h, chunk): step = softplus(dt + bias), cs = cumsum(step * A), and
+//               S = sum_l step_l e^{T - cs_l} x_l (x) B_l   (P x N); in the same launch, per
+//               (b, chunk, group), the lower tiles of CB = C . B^T (shared by the heads)
 //   state_pass  per (b, h), element-wise over P x N, sequential over chunks:
 //               entering state of every chunk, and the final state
 //   chunk_scan  per (b, h, chunk, 64-token tile), or per (b, h, chunk) for 16-bit inputs
@@ -21,82 +21,6 @@ namespace mko {
 namespace ssd {
 
 // ---------------------------------------------------------------- kernels
-
-__global__ void __launch_bounds__(256) prep(Geo g, Ptrs p) {
-  __shared__ float wsum[4];
-  const int c = blockIdx.x;
-  const int64_t h = blockIdx.y, b = blockIdx.z;
-  const int l = threadIdx.x;
-  const int64_t t = static_cast<int64_t>(c) * g.q + l;
-  float del = 0.0f;
-  if (l < g.q && t < g.length) {
-    float raw = load_one(p.dt, g.dt_dtype, (b * g.length + t) * g.nheads + h);
-    if (p.bias) raw += p.bias[h];
-    del = g.softplus ? softplus(raw) : raw;
-  }
-  float v = del * p.A[h];
-  // inclusive scan over the workgroup: wavefront butterflies, then wavefront offsets
-  for (int off = 1; off < kWave; off <<= 1) {
-    const float n = __shfl_up(v, off);
-    if ((l & 63) >= off) v += n;
-  }
-  if ((l & 63) == 63) wsum[l >> 6] = v;
-  __syncthreads();
-  for (int w = 0; w < (l >> 6); ++w) v += wsum[w];
-  if (l < g.q) {
-    const int64_t o = ((b * g.nheads + h) * g.nc + c) * g.q + l;
-    p.dl[o] = del;
-    p.cs[o] = v;
-  }
-}
-
-template <typename TM, bool VEC>
-__global__ void __launch_bounds__(256) cb_kernel(Geo g, Ptrs p) {
-  constexpr int TE = LdsTile<TM>::elems;
-  constexpr int NB = kStageBufs<TM>;
-  __shared__ __align__(16) TM sbuf[NB][2 * TE];
-  // lower-triangular tile (i, j), j <= i
-  const WgId id = wg_id(g.qb * (g.qb + 1) / 2, g.nc * g.ngroups);
-  const int idx = id.x;
-  int i = 0;
-  while ((i + 1) * (i + 2) / 2 <= idx) ++i;
-  const int j = idx - i * (i + 1) / 2;
-  const int c = id.y / g.ngroups;
-  const int64_t gg = id.y % g.ngroups, b = id.z;
-  const int lane = threadIdx.x & 63;
-  int wm, wn;
-  quadrant(threadIdx.x >> 6, wm, wn);
-  const int r0 = blk_r0(), c0 = blk_c0();
-  const int64_t tc = static_cast<int64_t>(c) * g.q;
-  const TM* Cm = static_cast<const TM*>(p.C);
-  const TM* Bm = static_cast<const TM*>(p.B);
-  struct Regs {
-    V8<TM> c[2], b[2];
-  };
-  auto fetch = [&](int k, Regs& r) {
-    load_bw<TM, VEC>(g, Cm, b, tc + 64 * i, gg, 64 * k, r.c);
-    load_bw<TM, VEC>(g, Bm, b, tc + 64 * j, gg, 64 * k, r.b);
-  };
-  auto put = [&](int k, Regs& r) {
-    TM* buf = sbuf[k % NB];
-    put_raw<TM, false>(buf, r0, c0, r.c[0], r.c[1]);       // A[l][n] = C_l[n]
-    put_raw<TM, false>(buf + TE, r0, c0, r.b[0], r.b[1]);  // Bt[s][n] = B_s[n]
-  };
-  f32x16 acc;
-  zero(acc);
-  auto mma = [&](int k) { mma_tile<TM>(acc, sbuf[k % NB], sbuf[k % NB] + TE, wm, wn, lane, 64); };
-  Regs ra;
-  if constexpr (NB == 1) {
-    pipeline1(g.nnt, ra, fetch, put, mma);
-  } else {
-    Regs rb;
-    pipeline2(g.nnt, ra, rb, fetch, put, mma);
-  }
-  TM* out = static_cast<TM*>(p.cb) + ((b * g.nc + c) * g.ngroups + gg) * g.q * g.q;
-#pragma unroll
-  for (int r = 0; r < 16; ++r)
-    out[(64 * i + acc_row(wm, lane, r)) * g.q + 64 * j + acc_col(wn, lane)] = from_f32<TM>(acc[r]);
-}
 
 // Entering state of every chunk (in place over the local states) and the final
 // state, 8 consecutive state elements per thread, sequential over the chunks.
@@ -595,9 +519,6 @@ Ptrs base_ptrs(const mko_ssd_params* prm) {
 template <typename TM, bool VEC>
 static void launch_fwd_t(const Geo& g, const Ptrs& q, hipStream_t s) {
   const unsigned bh = static_cast<unsigned>(g.batch * g.nheads);
-  MKO_TIMED("ssd_prep", s, prep<<<dim3(g.nc, g.nheads, g.batch), 256, 0, s>>>(g, q));
-  MKO_TIMED("ssd_cb", s,
-            cb_kernel<TM, VEC><<<dim3(g.qb * (g.qb + 1) / 2 * g.nc * g.ngroups * g.batch), 256, 0, s>>>(g, q));
   launch_chunk_state<TM, VEC, false>(g, q, q.states, s);
   MKO_TIMED("ssd_state_pass", s,
             state_pass<TM><<<dim3(static_cast<unsigned>((g.headdim * g.dstate + 2047) / 2048), bh), 256, 0, s>>>(

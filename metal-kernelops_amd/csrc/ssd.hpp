@@ -174,6 +174,84 @@ __device__ __forceinline__ void scale8(const V8<TM>& v, float s, float (&f)[8]) 
   for (int k = 0; k < 8; ++k) f[k] *= s;
 }
 
+// One token of a chunk a thread: the step size softplus(dt + bias) of token threadIdx.x (0 past
+// the chunk or the sequence), and in cs its inclusive cumulative sum of step * A over the chunk.
+// wsum: 4 floats of LDS.
+__device__ __forceinline__ float chunk_steps(const Geo& g, const Ptrs& p, int64_t b, int64_t h, int c, float* wsum,
+                                             float& cs) {
+  const int l = threadIdx.x;
+  const int64_t t = static_cast<int64_t>(c) * g.q + l;
+  float del = 0.0f;
+  if (l < g.q && t < g.length) {
+    float raw = load_one(p.dt, g.dt_dtype, (b * g.length + t) * g.nheads + h);
+    if (p.bias) raw += p.bias[h];
+    del = g.softplus ? softplus(raw) : raw;
+  }
+  float v = del * p.A[h];
+  // inclusive scan over the workgroup: wavefront butterflies, then wavefront offsets
+  for (int off = 1; off < kWave; off <<= 1) {
+    const float n = __shfl_up(v, off);
+    if ((l & 63) >= off) v += n;
+  }
+  if ((l & 63) == 63) wsum[l >> 6] = v;
+  __syncthreads();
+  for (int w = 0; w < (l >> 6); ++w) v += wsum[w];
+  __syncthreads();
+  cs = v;
+  return del;
+}
+
+// One lower tile (i, j), j <= i, of a (batch, chunk, group)'s C.B^T, shared by the group's heads:
+// workgroup w of total.
+template <typename TM, bool VEC>
+__device__ __forceinline__ void cb_tile(const Geo& g, const Ptrs& p, int64_t w, int64_t total, TM* sbuf) {
+  constexpr int TE = LdsTile<TM>::elems;
+  constexpr int NB = kStageBufs<TM>;
+  const WgId id = wg_id(g.qb * (g.qb + 1) / 2, g.nc * g.ngroups, w, total);
+  const int idx = id.x;
+  int i = 0;
+  while ((i + 1) * (i + 2) / 2 <= idx) ++i;
+  const int j = idx - i * (i + 1) / 2;
+  const int c = id.y / g.ngroups;
+  const int64_t gg = id.y % g.ngroups, b = id.z;
+  const int lane = threadIdx.x & 63;
+  int wm, wn;
+  quadrant(threadIdx.x >> 6, wm, wn);
+  const int r0 = blk_r0(), c0 = blk_c0();
+  const int64_t tc = static_cast<int64_t>(c) * g.q;
+  const TM* Cm = static_cast<const TM*>(p.C);
+  const TM* Bm = static_cast<const TM*>(p.B);
+  struct Regs {
+    V8<TM> c[2], b[2];
+  };
+  auto fetch = [&](int k, Regs& r) {
+    load_bw<TM, VEC>(g, Cm, b, tc + 64 * i, gg, 64 * k, r.c);
+    load_bw<TM, VEC>(g, Bm, b, tc + 64 * j, gg, 64 * k, r.b);
+  };
+  auto put = [&](int k, Regs& r) {
+    TM* buf = sbuf + (k % NB) * 2 * TE;
+    put_raw<TM, false>(buf, r0, c0, r.c[0], r.c[1]);       // A[l][n] = C_l[n]
+    put_raw<TM, false>(buf + TE, r0, c0, r.b[0], r.b[1]);  // Bt[s][n] = B_s[n]
+  };
+  f32x16 acc;
+  zero(acc);
+  auto mma = [&](int k) {
+    const TM* buf = sbuf + (k % NB) * 2 * TE;
+    mma_tile<TM>(acc, buf, buf + TE, wm, wn, lane, 64);
+  };
+  Regs ra;
+  if constexpr (NB == 1) {
+    pipeline1(g.nnt, ra, fetch, put, mma);
+  } else {
+    Regs rb;
+    pipeline2(g.nnt, ra, rb, fetch, put, mma);
+  }
+  TM* out = static_cast<TM*>(p.cb) + ((b * g.nc + c) * g.ngroups + gg) * g.q * g.q;
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    out[(64 * i + acc_row(wm, lane, r)) * g.q + 64 * j + acc_col(wn, lane)] = from_f32<TM>(acc[r]);
+}
+
 // out[p][n] = sum_l s1(l) X(l, p) Y(l, n) over the chunk, for one 64-row d_head tile
 // and two 64-column d_state tiles, stored in TM.
 //   FWD: X = x, s1 = step e^{T - cs}, Y = B  -> local chunk state
@@ -185,15 +263,26 @@ __device__ __forceinline__ void scale8(const V8<TM>& v, float s, float (&f)[8]) 
 // QB > 0: the chunk has QB 64-token tiles (a compile-time stage count, with the loads of
 // up to three stages in flight); QB = 0: qb at run time, two stages in flight (fp32: one, on a
 // single buffer, see kStageBufs; 4 x 1024 tokens, 32 heads, d_state 128: 57 -> 43 us)
+// The forward's launch also has, as its first ncb workgroups, the C.B^T tiles (cb_tile): they
+// wait for nothing and only chunk_scan reads them.  And it forms the chunk's step sizes and
+// decay exponents itself, one token a thread.  As three launches: 11 + 9 + 58 us at 4 x 4096
+// tokens, 64 heads, 65 together; a 1 x 1999-token prompt of 24 heads 38 -> 32 us.
 template <typename TM, bool VEC, bool BWD, int QB = 0>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-chunk_state(Geo g, Ptrs p, void* out_) {
+chunk_state(Geo g, Ptrs p, void* out_, int ncb) {
   constexpr int LD = compact_ld<TM>();  // LDS bounds this kernel: the compact tiles
   constexpr int TE = LdsTile<TM, LD>::elems;
   constexpr int NB = kStageBufs<TM>;
   __shared__ __align__(16) TM sbuf[NB][3 * TE];
   __shared__ float s1[256];
-  const WgId id = wg_id(g.npt * g.nnp, g.nc);
+  static_assert(sizeof(sbuf) >= kStageBufs<TM> * 2 * LdsTile<TM>::elems * sizeof(TM), "cb_tile's operands fit");
+  if constexpr (!BWD) {
+    if (static_cast<int>(blockIdx.x) < ncb) {
+      cb_tile<TM, VEC>(g, p, blockIdx.x, ncb, &sbuf[0][0]);
+      return;
+    }
+  }
+  const WgId id = wg_id(g.npt * g.nnp, g.nc, blockIdx.x - ncb, gridDim.x - ncb);
   const int pt = id.x / g.nnp, np = id.x % g.nnp;
   const int c = id.y;
   const int64_t bh = id.z, b = bh / g.nheads, h = bh % g.nheads, gg = h / g.hpg;
@@ -202,10 +291,21 @@ chunk_state(Geo g, Ptrs p, void* out_) {
   quadrant(threadIdx.x >> 6, wm, wn);
   const int r0 = blk_r0(), c0 = blk_c0();
   const int64_t so = (bh * g.nc + c) * g.q;
-  const float T = p.cs[so + g.q - 1];
-  for (int l = threadIdx.x; l < g.q; l += 256) {
-    const bool ok = static_cast<int64_t>(c) * g.q + l < g.length;
-    s1[l] = !ok ? 0.0f : (BWD ? fast_exp(p.cs[so + l]) : p.dl[so + l] * fast_exp(T - p.cs[so + l]));
+  if constexpr (BWD) {
+    for (int l = threadIdx.x; l < g.q; l += 256)
+      s1[l] = static_cast<int64_t>(c) * g.q + l < g.length ? fast_exp(p.cs[so + l]) : 0.0f;
+  } else {
+    float cs;
+    const float del = chunk_steps(g, p, b, h, c, s1, cs);
+    if (id.x == 0 && static_cast<int>(threadIdx.x) < g.q) {
+      p.dl[so + threadIdx.x] = del;
+      p.cs[so + threadIdx.x] = cs;
+    }
+    s1[threadIdx.x] = cs;
+    __syncthreads();
+    const float T = s1[g.q - 1];
+    __syncthreads();
+    s1[threadIdx.x] = del * fast_exp(T - cs);  // 0 past the sequence, where the step is
   }
   const TM* X = static_cast<const TM*>(BWD ? p.gy : p.x);
   const TM* Y = static_cast<const TM*>(BWD ? p.C : p.B);
@@ -269,15 +369,16 @@ chunk_state(Geo g, Ptrs p, void* out_) {
 
 template <typename TM, bool VEC, bool BWD>
 inline void launch_chunk_state(const Geo& g, const Ptrs& q, void* out, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(g.npt * g.nnp * g.nc * g.batch * g.nheads));
+  const int ncb = BWD ? 0 : static_cast<int>(g.qb * (g.qb + 1) / 2 * g.nc * g.ngroups * g.batch);
+  const dim3 grid(static_cast<unsigned>(ncb + g.npt * g.nnp * g.nc * g.batch * g.nheads));
   const char* name = BWD ? "ssd_chunk_state_bwd" : "ssd_chunk_state";
   if constexpr (sizeof(TM) == 2) {
     if (g.qb == 4) {
-      MKO_TIMED(name, s, chunk_state<TM, VEC, BWD, 4><<<grid, 256, 0, s>>>(g, q, out));
+      MKO_TIMED(name, s, chunk_state<TM, VEC, BWD, 4><<<grid, 256, 0, s>>>(g, q, out, ncb));
       return;
     }
   }
-  MKO_TIMED(name, s, chunk_state<TM, VEC, BWD><<<grid, 256, 0, s>>>(g, q, out));
+  MKO_TIMED(name, s, chunk_state<TM, VEC, BWD><<<grid, 256, 0, s>>>(g, q, out, ncb));
 }
 
 // Loads cs and step of a whole chunk into LDS (q <= 256 values each), and the column
