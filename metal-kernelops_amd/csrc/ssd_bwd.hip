@@ -21,9 +21,9 @@
 // sides use the same rounded operands (gy and u as the matrix cores see them) and
 // the cancellation between them is exact up to fp32 accumulation.
 //   reduce      dA, ddt_bias, dD
-// Every partial sum is reduced in a fixed order: the backward is deterministic.  dcb runs on
-// a second stream beside state_rev, du, dbc_state, finish and reduce (launch_bwd_t), and
-// dbc_final, which reads its partials, runs last.
+// Every partial sum is reduced in a fixed order: the backward is deterministic.  finish runs in
+// dbc_state's launch and reduce in dbc_final's.  dcb runs on a second stream beside state_rev,
+// du and dbc_state (launch_bwd_t), and dbc_final, which reads its partials, runs last.
 #include <algorithm>
 #include <mutex>
 #include <vector>
@@ -1064,17 +1064,144 @@ dcb_kernel(Geo g, BwdPlan pl, Ptrs p) {
     out[(64 * i + acc_row(wm, lane, r)) * g.q + 64 * j + acc_col(wn, lane)] = dacc[r];
 }
 
+// Per (b, h, chunk), one thread per token in reverse order: d cs, its reverse
+// cumulative sum, d step, ddt, and the dA / ddt_bias partials.
+__device__ __forceinline__ void finish(const Geo& g, const BwdPlan& pl, const Ptrs& p, int64_t w) {
+  __shared__ float wsum[4];
+  const int c = static_cast<int>(w % g.nc);
+  const int64_t bh = w / g.nc, b = bh / g.nheads, h = bh % g.nheads;
+  const int tid = threadIdx.x;
+  const bool active = tid < g.q;
+  const int l = g.q - 1 - tid;
+  const int64_t so = (bh * g.nc + c) * g.q;
+  float dcs = 0.0f, dsxv = 0.0f, del = 0.0f, tau = 0.0f;
+  if (active) {
+    for (int pt = 0; pt < g.npt; ++pt) {
+      const int64_t o = ((bh * g.nc + c) * g.npt + pt) * g.q + l;
+      dcs += p.ya[o] - p.ut[o];
+      dsxv += p.dsx[o];
+      tau += p.tau[o];
+    }
+    del = p.dl[so + l];
+  }
+  // d T = sum_s tau_s + e^T <G, S_in>, at the chunk's last position
+  const float tau_sum = block_sum(tau, wsum);
+  if (active && l == g.q - 1) {
+    dcs += tau_sum;
+    for (int k = 0; k < pl.nblk; ++k) dcs += p.dT[(bh * g.nc + c) * pl.nblk + k];
+  }
+  __syncthreads();
+  // inclusive scan in thread order = suffix sum over the chunk positions
+  float v = dcs;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const float n = __shfl_up(v, off);
+    if ((tid & 63) >= off) v += n;
+  }
+  if ((tid & 63) == 63) wsum[tid >> 6] = v;
+  __syncthreads();
+  for (int w = 0; w < (tid >> 6); ++w) v += wsum[w];
+  const float rcs = v;
+  const float ddel = fmaf(p.A[h], rcs, dsxv);
+  const int64_t t = static_cast<int64_t>(c) * g.q + l;
+  float dd = 0.0f;
+  if (active && t < g.length) {
+    const int64_t o = (b * g.length + t) * g.nheads + h;
+    float raw = load_one(p.dt, g.dt_dtype, o);
+    if (p.bias) raw += p.bias[h];
+    dd = g.softplus ? ddel * softplus_grad(raw) : ddel;
+    store_one(p.ddt, g.dt_dtype, o, dd);
+  }
+  __syncthreads();
+  const float sa = block_sum(del * rcs, wsum);
+  const float sb = block_sum(dd, wsum);
+  if (tid == 0) {
+    p.pA[bh * g.nc + c] = sa;
+    p.pbias[bh * g.nc + c] = sb;
+  }
+}
+
+// dA, ddt_bias and dD of head h.
+__device__ __forceinline__ void reduce_head(const Geo& g, const Ptrs& p, int64_t h) {
+  __shared__ float wsum[4];
+  const int tid = threadIdx.x;
+  const int64_t nbc = g.batch * g.nc;
+  float sa = 0.0f, sb = 0.0f;
+  for (int64_t k = tid; k < nbc; k += 256) {
+    const int64_t o = ((k / g.nc) * g.nheads + h) * g.nc + k % g.nc;
+    sa += p.pA[o];
+    sb += p.pbias[o];
+  }
+  sa = block_sum(sa, wsum);
+  sb = block_sum(sb, wsum);
+  if (tid == 0) {
+    p.dA[h] = sa;
+    if (p.dbias) p.dbias[h] = sb;
+  }
+  if (!p.dD) return;
+  // dD: (b, chunk, tile) partial rows; 64 columns x 4 row groups per pass
+  __shared__ float part[4][64];
+  const int64_t nrow = nbc * g.qb;
+  const int col = tid & 63, grp = tid >> 6;
+  float hsum = 0.0f;
+  for (int pt = 0; pt < g.npt; ++pt) {
+    const int64_t pc = static_cast<int64_t>(pt) * 64 + col;
+    // rows grp, grp + 4, ... in 16 chains, so that 16 loads are in flight per thread
+    float sv[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sv[e] = 0.0f;
+    if (pc < g.headdim) {
+      const float* q = p.pdD + h * g.headdim + pc;
+      const int64_t stride = g.nheads * g.headdim;
+      int64_t k = grp;
+      for (; k + 60 < nrow; k += 64) {
+        float v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = q[(k + 4 * e) * stride];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sv[e] += v[e];
+      }
+      for (; k < nrow; k += 4) sv[0] += q[k * stride];
+    }
+#pragma unroll
+    for (int w = 8; w >= 1; w >>= 1)
+#pragma unroll
+      for (int e = 0; e < w; ++e) sv[e] += sv[e + w];
+    __syncthreads();
+    part[grp][col] = sv[0];
+    __syncthreads();
+    if (tid < 64 && pc < g.headdim) {
+      const float tot = (part[0][col] + part[1][col]) + (part[2][col] + part[3][col]);
+      if (g.d_per_row)
+        p.dD[h * g.headdim + pc] = tot;
+      else
+        hsum += tot;
+    }
+  }
+  if (!g.d_per_row) {
+    hsum = block_sum(hsum, wsum);
+    if (tid == 0) p.dD[h] = hsum;
+  }
+}
+
+__global__ void __launch_bounds__(256) reduce_params(Geo g, Ptrs p) { reduce_head(g, p, blockIdx.x); }
+
 // State terms of dB (which 0: sum_h e^{T - cs_s} step_s x_s G) and dC (which 1:
 // sum_h e^{cs_l} gy_l S_in) for one 64-token tile and two d_state tiles, over a
-// block of the group's heads.
+// block of the group's heads.  The launch's workgroups from nst_wgs on run finish, whose short
+// dependent loads then overlap these products (at 4 x 4096 tokens, 64 heads, 86 + 20 us as two
+// launches, 104 as one, and one launch gap fewer).
 template <typename TM, bool VEC>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
-dbc_state(Geo g, BwdPlan pl, Ptrs p) {
+dbc_state(Geo g, BwdPlan pl, Ptrs p, int nst_wgs) {
   constexpr int LD = compact_ld<TM>();  // LDS bounds this kernel: the compact tiles
   constexpr int TE = LdsTile<TM, LD>::elems;
   constexpr int NB = kStageBufs<TM>;
   __shared__ __align__(16) TM sbuf[NB][3 * TE];
-  const WgId id = wg_id(g.qb * g.nnp * 2 * pl.hb2, g.nc * g.ngroups);
+  if (static_cast<int>(blockIdx.x) >= nst_wgs) {
+    finish(g, pl, p, blockIdx.x - nst_wgs);
+    return;
+  }
+  const WgId id = wg_id(g.qb * g.nnp * 2 * pl.hb2, g.nc * g.ngroups, blockIdx.x, nst_wgs);
   int idx = id.x;
   const int hb = idx % pl.hb2;
   idx /= pl.hb2;
@@ -1153,13 +1280,19 @@ dbc_state(Geo g, BwdPlan pl, Ptrs p) {
 }
 
 // dC = dCB B (which 1) and dB = dCB^T C (which 0) for one 64-token tile and two
-// d_state tiles, plus the head-block partials of the state terms.
+// d_state tiles, plus the head-block partials of the state terms.  The launch's first nheads
+// workgroups are reduce_head's.
 template <typename TM, bool VEC>
 __global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
   constexpr int TE = LdsTile<TM>::elems;
   constexpr int NB = kStageBufs<TM>;
   __shared__ __align__(16) TM sbuf[NB][3 * TE];
-  const WgId id = wg_id(g.qb * g.nnp * 2, g.nc * g.ngroups);
+  const int heads = static_cast<int>(g.nheads);
+  if (static_cast<int>(blockIdx.x) < heads) {
+    reduce_head(g, p, blockIdx.x);
+    return;
+  }
+  const WgId id = wg_id(g.qb * g.nnp * 2, g.nc * g.ngroups, blockIdx.x - heads, gridDim.x - heads);
   int idx = id.x;
   const int which = idx % 2;
   idx /= 2;
@@ -1252,125 +1385,6 @@ __global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
       }
     }
     store_bw<TM, VEC>(g, out, b, t0, gg, nn0 + 64 * half, v[0], v[1]);
-  }
-}
-
-// Per (b, h, chunk), one thread per token in reverse order: d cs, its reverse
-// cumulative sum, d step, ddt, and the dA / ddt_bias partials.
-__global__ void __launch_bounds__(256) finish(Geo g, BwdPlan pl, Ptrs p) {
-  __shared__ float wsum[4];
-  const int c = blockIdx.x;
-  const int64_t h = blockIdx.y, b = blockIdx.z, bh = b * g.nheads + h;
-  const int tid = threadIdx.x;
-  const bool active = tid < g.q;
-  const int l = g.q - 1 - tid;
-  const int64_t so = (bh * g.nc + c) * g.q;
-  float dcs = 0.0f, dsxv = 0.0f, del = 0.0f, tau = 0.0f;
-  if (active) {
-    for (int pt = 0; pt < g.npt; ++pt) {
-      const int64_t o = ((bh * g.nc + c) * g.npt + pt) * g.q + l;
-      dcs += p.ya[o] - p.ut[o];
-      dsxv += p.dsx[o];
-      tau += p.tau[o];
-    }
-    del = p.dl[so + l];
-  }
-  // d T = sum_s tau_s + e^T <G, S_in>, at the chunk's last position
-  const float tau_sum = block_sum(tau, wsum);
-  if (active && l == g.q - 1) {
-    dcs += tau_sum;
-    for (int k = 0; k < pl.nblk; ++k) dcs += p.dT[(bh * g.nc + c) * pl.nblk + k];
-  }
-  __syncthreads();
-  // inclusive scan in thread order = suffix sum over the chunk positions
-  float v = dcs;
-  for (int off = 1; off < kWave; off <<= 1) {
-    const float n = __shfl_up(v, off);
-    if ((tid & 63) >= off) v += n;
-  }
-  if ((tid & 63) == 63) wsum[tid >> 6] = v;
-  __syncthreads();
-  for (int w = 0; w < (tid >> 6); ++w) v += wsum[w];
-  const float rcs = v;
-  const float ddel = fmaf(p.A[h], rcs, dsxv);
-  const int64_t t = static_cast<int64_t>(c) * g.q + l;
-  float dd = 0.0f;
-  if (active && t < g.length) {
-    const int64_t o = (b * g.length + t) * g.nheads + h;
-    float raw = load_one(p.dt, g.dt_dtype, o);
-    if (p.bias) raw += p.bias[h];
-    dd = g.softplus ? ddel * softplus_grad(raw) : ddel;
-    store_one(p.ddt, g.dt_dtype, o, dd);
-  }
-  __syncthreads();
-  const float sa = block_sum(del * rcs, wsum);
-  const float sb = block_sum(dd, wsum);
-  if (tid == 0) {
-    p.pA[bh * g.nc + c] = sa;
-    p.pbias[bh * g.nc + c] = sb;
-  }
-}
-
-__global__ void __launch_bounds__(256) reduce_params(Geo g, BwdPlan pl, Ptrs p) {
-  __shared__ float wsum[4];
-  const int64_t h = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int64_t nbc = g.batch * g.nc;
-  float sa = 0.0f, sb = 0.0f;
-  for (int64_t k = tid; k < nbc; k += 256) {
-    const int64_t o = ((k / g.nc) * g.nheads + h) * g.nc + k % g.nc;
-    sa += p.pA[o];
-    sb += p.pbias[o];
-  }
-  sa = block_sum(sa, wsum);
-  sb = block_sum(sb, wsum);
-  if (tid == 0) {
-    p.dA[h] = sa;
-    if (p.dbias) p.dbias[h] = sb;
-  }
-  if (!p.dD) return;
-  // dD: (b, chunk, tile) partial rows; 64 columns x 4 row groups per pass
-  __shared__ float part[4][64];
-  const int64_t nrow = nbc * g.qb;
-  const int col = tid & 63, grp = tid >> 6;
-  float hsum = 0.0f;
-  for (int pt = 0; pt < g.npt; ++pt) {
-    const int64_t pc = static_cast<int64_t>(pt) * 64 + col;
-    // rows grp, grp + 4, ... in 16 chains, so that 16 loads are in flight per thread
-    float sv[16];
-#pragma unroll
-    for (int e = 0; e < 16; ++e) sv[e] = 0.0f;
-    if (pc < g.headdim) {
-      const float* q = p.pdD + h * g.headdim + pc;
-      const int64_t stride = g.nheads * g.headdim;
-      int64_t k = grp;
-      for (; k + 60 < nrow; k += 64) {
-        float v[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = q[(k + 4 * e) * stride];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) sv[e] += v[e];
-      }
-      for (; k < nrow; k += 4) sv[0] += q[k * stride];
-    }
-#pragma unroll
-    for (int w = 8; w >= 1; w >>= 1)
-#pragma unroll
-      for (int e = 0; e < w; ++e) sv[e] += sv[e + w];
-    __syncthreads();
-    part[grp][col] = sv[0];
-    __syncthreads();
-    if (tid < 64 && pc < g.headdim) {
-      const float tot = (part[0][col] + part[1][col]) + (part[2][col] + part[3][col]);
-      if (g.d_per_row)
-        p.dD[h * g.headdim + pc] = tot;
-      else
-        hsum += tot;
-    }
-  }
-  if (!g.d_per_row) {
-    hsum = block_sum(hsum, wsum);
-    if (tid == 0) p.dD[h] = hsum;
   }
 }
 
@@ -1517,7 +1531,7 @@ int stream_wait(hipStream_t from, hipStream_t to, hipEvent_t e) {
 
 // The kernels after the gate, in two streams.  dcb reads only gy and the forward's inputs
 // and writes only partials that dbc_final reads, so the side stream runs it as soon as the
-// gate is done, beside state_rev, du, dbc_state, finish and reduce_params on s, and s waits
+// gate is done, beside state_rev, du and dbc_state (with finish) on s, and s waits
 // for it just before dbc_final.  Alone at 4 x 4096 tokens and 64 heads, dcb's 640 long
 // workgroups leave about 40% of the workgroup slots empty for 0.12 ms.  (dbc_state could
 // follow it there once state_rev is done; it runs faster on s, where it does not compete with
@@ -1559,11 +1573,9 @@ int launch_bwd_t(const Geo& g, const BwdPlan& pl, const Ptrs& q, hipStream_t s) 
   MKO_TIMED("ssd_state_rev", s, state_rev<TM><<<dim3(pl.nblk, bh), 256, 0, s>>>(g, pl, q));
   launch_du<TM, VEC>(g, pl, q, s);
   if (!join) dcb(s);
+  const unsigned nst_wgs = g.qb * g.nnp * 2 * pl.hb2 * ncg * nb;
   MKO_TIMED("ssd_dbc_state", s,
-            dbc_state<TM, VEC><<<dim3(g.qb * g.nnp * 2 * pl.hb2 * ncg * nb), 256, 0, s>>>(g, pl, q));
-  MKO_TIMED("ssd_finish", s,
-            finish<<<dim3(g.nc, static_cast<unsigned>(g.nheads), nb), 256, 0, s>>>(g, pl, q));
-  MKO_TIMED("ssd_reduce", s, reduce_params<<<dim3(static_cast<unsigned>(g.nheads)), 256, 0, s>>>(g, pl, q));
+            dbc_state<TM, VEC><<<dim3(nst_wgs + g.nc * bh), 256, 0, s>>>(g, pl, q, static_cast<int>(nst_wgs)));
   if (join) {
     const hipError_t e = hipStreamWaitEvent(s, join, 0);
     if (e != hipSuccess) {
@@ -1571,7 +1583,8 @@ int launch_bwd_t(const Geo& g, const BwdPlan& pl, const Ptrs& q, hipStream_t s) 
       return MKO_ELAUNCH;
     }
   }
-  MKO_TIMED("ssd_dbc_final", s, dbc_final<TM, VEC><<<dim3(g.qb * g.nnp * 2 * ncg * nb), 256, 0, s>>>(g, pl, q));
+  MKO_TIMED("ssd_dbc_final", s,
+            dbc_final<TM, VEC><<<dim3(static_cast<unsigned>(g.nheads) + g.qb * g.nnp * 2 * ncg * nb), 256, 0, s>>>(g, pl, q));
   return MKO_OK;
 }
 
@@ -1646,7 +1659,7 @@ extern "C" int mko_ssd_bwd(const mko_ssd_params* prm, void* stream) {
       else if (g.x_dtype == MKO_BF16) MKO_TIMED("ssd_state_rev", s, state_rev<bf16><<<grid, 256, 0, s>>>(g, pl, q));
       else MKO_TIMED("ssd_state_rev", s, state_rev<_Float16><<<grid, 256, 0, s>>>(g, pl, q));
     }
-    MKO_TIMED("ssd_reduce", s, reduce_params<<<dim3(static_cast<unsigned>(g.nheads)), 256, 0, s>>>(g, pl, q));
+    MKO_TIMED("ssd_reduce", s, reduce_params<<<dim3(static_cast<unsigned>(g.nheads)), 256, 0, s>>>(g, q));
   }
   return mko_check_launch("ssd_bwd");
 }
