@@ -388,8 +388,8 @@ __global__ void __launch_bounds__(256) forward_il(Geo g, mko_conv1d_params p) {
 // walking forwards every lane formed those H slopes again (11 for 8 steps at K = 4).  The H
 // steps before a block come from lane l - 1 (lane 0: from lane 63's next block, which is in
 // flight two iterations ahead, or the steps before the segment).  Iterations past the row's end
-// are not run.  At 4 x 5120 x 4096, K 4, bf16, SiLU, 128 -> 110 us; 8 x 1536 x 384,
-// one iteration of a possible eight, 37 -> 18 us.
+// are not run.  At 4 x 5120 x 4096, K 4, bf16, SiLU, 115 -> 108 us; 8 x 1536 x 384,
+// one iteration of a possible eight, 34 -> 17 us.
 // The loop stays rolled: unrolled, its registers cost a wavefront per SIMD.
 // The taps' gradients are summed over the wavefront, which
 // lies in one row, and `finalize_il` adds the wavefronts' partials in order.
