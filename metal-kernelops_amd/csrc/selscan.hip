@@ -1921,8 +1921,9 @@ static int lane_chunks(const Geo& g) {
   return quads <= 384 && nblk >= 32 ? 16 : 4;
 }
 
-// Time chunks of the lane-per-state backward: the smallest power of two that gives every slot
-// of the chip (3 wavefronts on each of 1024 SIMDs) a wavefront, with at least four blocks each.
+// Time chunks of the lane-per-state backward: the smallest power of two that gives each of 1024
+// SIMDs 3 wavefronts, with at least four blocks each.  (bwd_lane holds four a SIMD since its LDS
+// and registers were cut; the figures are from before, and the line was not moved.)
 // A chunk costs its bwd_map and its own dA / dD / ddelta_bias partials.  us a backward with
 // 1 / 2 / 4 / 8 / 32 chunks, bf16: 5120 rows x 1024 steps 153 / 131 / 116 / 117 / 149, 1536 x 2048
 // 210 / 141 / 101 / 78 / 84, 384 x 3136 309 / 199 / 110 / 67 / 48, 8 x 1536 x 2048 413 / 436.
