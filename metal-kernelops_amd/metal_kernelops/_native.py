@@ -262,21 +262,34 @@ def code(dtype):
     return _DTYPE_CODE[dtype]
 
 
+def dense_op(name, impl):
+    """Registers ``impl`` as the custom op ``name``, its tensors dense: the dispatcher hands a
+    kernel a ZeroTensor as one element expanded to the shape, and the kernels read dense memory."""
+
+    def op(*args):
+        return impl(*(t.contiguous() if isinstance(t, torch.Tensor) else t for t in args))
+
+    return torch.library.custom_op(name, op, mutates_args=(), device_types="cuda",
+                                   schema=torch.library.infer_schema(impl, mutates_args=()))
+
+
 def plain_call(*tensors):
     """Whether a call on ``tensors`` (None among them allowed) is an ordinary eager one that no
     gradient, tracer or mode has to see, so that the implementation behind a custom op may be
     called without the dispatcher: its round trip costs 10-25 us of host time, as much as the
     kernels of a short prompt.  Not plain: grad mode with an input that requires grad, compiling
-    or tracing, tensor subclasses, dispatch or function modes, functorch transforms and
-    forward-mode levels; those go through the op, which does with them what it always did."""
+    or tracing, a profiler that is recording (it names the op), tensor subclasses, dispatch or
+    function modes, functorch transforms and forward-mode levels, and tensors whose values are not
+    what their memory holds (negated views, and those without memory: ZeroTensors, functional
+    wrappers, empty tensors); those go through the op, which does with them what it always did."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() \
             or torch._C._len_torch_function_stack() or torch._C._functorch.peek_interpreter_stack() is not None \
-            or torch.autograd.forward_ad._current_level >= 0:
+            or torch.autograd.forward_ad._current_level >= 0 or torch._C._autograd._profiler_enabled():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
         if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter)
-                              or (grad and t.requires_grad)):
+                              or (grad and t.requires_grad) or t.is_neg() or t.data_ptr() == 0):
             return False
     return True
 

@@ -113,7 +113,7 @@ def _conv1d_fwd_impl(x: Tensor, weight: Tensor, bias: Optional[Tensor], init: Op
     return out, final
 
 
-_conv1d_fwd = torch.library.custom_op("mko::conv1d_fwd", _conv1d_fwd_impl, mutates_args=(), device_types="cuda")
+_conv1d_fwd = nat.dense_op("mko::conv1d_fwd", _conv1d_fwd_impl)
 
 
 @_conv1d_fwd.register_fake
@@ -146,7 +146,7 @@ def _conv1d_bwd_impl(dout: Tensor, x: Tensor, weight: Tensor, bias: Optional[Ten
     return dx, dweight, dbias, dinit
 
 
-_conv1d_bwd = torch.library.custom_op("mko::conv1d_bwd", _conv1d_bwd_impl, mutates_args=(), device_types="cuda")
+_conv1d_bwd = nat.dense_op("mko::conv1d_bwd", _conv1d_bwd_impl)
 
 
 @_conv1d_bwd.register_fake

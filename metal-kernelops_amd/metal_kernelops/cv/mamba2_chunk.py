@@ -128,7 +128,7 @@ def _ssd_fwd_impl(x: Tensor, dt: Tensor, A: Tensor, B: Tensor, C: Tensor, D: Opt
     return y, final, saved
 
 
-_ssd_fwd = torch.library.custom_op("mko::ssd_fwd", _ssd_fwd_impl, mutates_args=(), device_types="cuda")
+_ssd_fwd = nat.dense_op("mko::ssd_fwd", _ssd_fwd_impl)
 
 
 @_ssd_fwd.register_fake
@@ -165,7 +165,7 @@ def _ssd_bwd_impl(dy: Tensor, dfinal: Optional[Tensor], x: Tensor, dt: Tensor, A
     return dx, ddt, dA, dB, dC, dD, dz, dbias, dinit
 
 
-_ssd_bwd = torch.library.custom_op("mko::ssd_bwd", _ssd_bwd_impl, mutates_args=(), device_types="cuda")
+_ssd_bwd = nat.dense_op("mko::ssd_bwd", _ssd_bwd_impl)
 
 
 @_ssd_bwd.register_fake

@@ -82,7 +82,7 @@ def selscan_fwd_impl(u: Tensor, delta: Tensor, A: Tensor, B: Tensor, C: Tensor, 
     return out, states
 
 
-_selscan_fwd = torch.library.custom_op("mko::selscan_fwd", selscan_fwd_impl, mutates_args=(), device_types="cuda")
+_selscan_fwd = nat.dense_op("mko::selscan_fwd", selscan_fwd_impl)
 
 
 @_selscan_fwd.register_fake
@@ -127,7 +127,7 @@ def selscan_bwd_impl(dout: Tensor, u: Tensor, delta: Tensor, A: Tensor, B: Tenso
     return du, ddelta, dA, dB, dC, dD, dz, dbias
 
 
-_selscan_bwd = torch.library.custom_op("mko::selscan_bwd", selscan_bwd_impl, mutates_args=(), device_types="cuda")
+_selscan_bwd = nat.dense_op("mko::selscan_bwd", selscan_bwd_impl)
 
 
 @_selscan_bwd.register_fake

@@ -1,6 +1,7 @@
-"""Which calls skip the dispatcher: ordinary eager ones only.  Under a dispatch mode, compilation,
-a functorch transform, a forward-mode level or a backward that is itself recorded, the operators go
-through their custom ops, and both ways give the same results."""
+"""Which calls skip the dispatcher: ordinary eager ones only.  Under a dispatch mode, a profiler,
+compilation, a functorch transform, a forward-mode level or a backward that is itself recorded, and
+on tensors whose memory does not hold their values, the operators go through their custom ops, and
+both ways give the same results."""
 
 import pytest
 import torch
@@ -47,6 +48,27 @@ def test_plain_call_rules():
         assert not nat.plain_call(t, t.as_subclass(Sub))
 
 
+def test_tensors_not_read_from_memory_are_not_plain():
+    # The dispatcher materialises these before a kernel sees them; their memory holds the negated
+    # values, or nothing.
+    t = torch.ones(3)
+    odd = {"negated": torch._neg_view(t), "zero": torch._efficientzerotensor((3,)),
+           "functional": torch._to_functional_tensor(t), "meta": t.to("meta")}
+    assert odd["negated"].contiguous().is_neg()  # a dense layout alone does not materialise it
+    with torch.no_grad():
+        for name, v in odd.items():
+            assert not nat.plain_call(t, v), name
+
+
+def test_a_recording_profiler_sees_the_op():
+    t = torch.ones(3)
+    with torch.no_grad():
+        assert nat.plain_call(t)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+            assert not nat.plain_call(t)
+        assert nat.plain_call(t)
+
+
 def _calls():
     from metal_kernelops import selective_scan
     from metal_kernelops.cv import causal_conv1d_fn, mamba2_chunk_scan
@@ -84,3 +106,32 @@ def test_modes_still_see_the_op(name):
     grads = torch.autograd.grad(fn(*leaves), leaves, dy, create_graph=True)
     with pytest.raises(RuntimeError):
         torch.autograd.grad(grads[0].sum(), leaves[:1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["selscan", "ssd", "conv1d"])
+def test_negated_views_and_zero_tensors_are_materialised(name):
+    fn, args = _calls()[name]
+    plain = [-args[0]] + args[1:]
+    zeros = [torch.zeros_like(args[0])] + args[1:]
+    with torch.no_grad():
+        assert torch.equal(fn(torch._neg_view(args[0]), *args[1:]), fn(*plain))
+        assert torch.equal(fn(torch._efficientzerotensor(tuple(args[0].shape), device=DEV), *args[1:]), fn(*zeros))
+    leaves = [t.clone().requires_grad_(True) for t in args]
+    dy = torch.randn_like(fn(*args))
+    got = torch.autograd.grad(fn(*leaves), leaves, torch._neg_view(dy))
+    want = torch.autograd.grad(fn(*leaves), leaves, -dy)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["selscan", "ssd", "conv1d"])
+def test_profiler_names_the_op(name):
+    fn, args = _calls()[name]
+    leaves = [t.clone().requires_grad_(True) for t in args]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        with torch.no_grad():
+            out = fn(*args)
+        torch.autograd.grad(fn(*leaves), leaves, torch.ones_like(out))
+    seen = [e.key for e in prof.key_averages()]
+    assert f"mko::{name}_fwd" in seen and f"mko::{name}_bwd" in seen, seen
