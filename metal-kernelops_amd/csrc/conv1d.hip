@@ -423,8 +423,9 @@ __global__ void __launch_bounds__(256) backward_il(Geo g, mko_conv1d_params p, f
   xe.load(g, xs, row, base + (last + 1) * kWave);
   de.load(g, ds, row, base + (last + 1) * kWave);
   xn.load(g, xs, row, block_at(last - 1));
-  // the gradient at step i of a window of z: dout act'(pre); dout, and so the gradient, is zero
-  // past the row
+  // the gradient at step i of a window of z: dout act'(pre).  dout is zero past the row, but the
+  // slope there may be none (z's last steps can take pre past fp32's range, or not be finite): a
+  // block past the row takes zeros for its look-back, and a ragged block's steps are cut off.
   auto grad = [&](const float* zz, float d) {
     float pre = bias;
 #pragma unroll
@@ -440,10 +441,14 @@ __global__ void __launch_bounds__(256) backward_il(Geo g, mko_conv1d_params p, f
 #pragma unroll
     for (int i = 0; i < H; ++i) {
       zz[i] = lane_of(xc[BS - H + i], kWave - 1);
+      if (VEC && base + (last + 1) * kWave >= g.nblk) zz[i] = 0.0f;
       zz[H + i] = xd[i];
     }
 #pragma unroll
-    for (int i = 0; i < H; ++i) right[i] = grad(zz + i, dd[i]);
+    for (int i = 0; i < H; ++i) {
+      right[i] = grad(zz + i, dd[i]);
+      if (!VEC && (base + (last + 1) * kWave) * BS + i >= g.length) right[i] = 0.0f;
+    }
   }
 #pragma unroll 1
   for (int k = last; k >= 0; --k) {
@@ -464,13 +469,17 @@ __global__ void __launch_bounds__(256) backward_il(Geo g, mko_conv1d_params p, f
         const float prev = __shfl_up(xc[BS - H + i], 1);
         const float edge = k > 0 ? lane_of(xl[BS - H + i], kWave - 1) : carry[i];
         zz[i] = lane == 0 ? edge : prev;
+        if (VEC && blk >= g.nblk) zz[i] = 0.0f;
       }
     }
 #pragma unroll
     for (int i = 0; i < BS; ++i) zz[H + i] = xc[i];
     float gg[BS + H];  // gg[i] = the gradient at t0 + i
 #pragma unroll
-    for (int i = 0; i < BS; ++i) gg[i] = grad(zz + i, dc[i]);
+    for (int i = 0; i < BS; ++i) {
+      gg[i] = grad(zz + i, dc[i]);
+      if (!VEC && t0 + i >= g.length) gg[i] = 0.0f;
+    }
 #pragma unroll
     for (int i = 0; i < H; ++i) {
       const float next = __shfl_down(gg[i], 1);

@@ -311,3 +311,24 @@ def test_backward_walk_edges(width, length, dtype):
     tol = 1e-4 if dtype == torch.float32 else 2e-2
     for name, g, r in zip(("x", "weight", "bias", "initial"), grads, want):
         assert rel(g, r) <= tol, (name, rel(g, r))
+
+
+# A pre-activation past the row's end is no part of the result.  The last step is large and its own
+# tap small, so that every step of the row is finite while the steps after it would overflow fp32,
+# where the SiLU has no slope: rows ending inside a block, with a block, with a wavefront's 64
+# blocks, and with its 4096 steps.
+@pytest.mark.gpu
+@pytest.mark.parametrize("length", [5, 8, 13, 512, 515, 4096, 4101])
+@pytest.mark.parametrize("width", [2, 4, 7])
+def test_backward_ignores_steps_past_the_row(width, length):
+    from metal_kernelops.cv import causal_conv1d_fn
+    x, dy = (make((2, 3, length), seed, dtype=torch.float32) for seed in (1, 2))
+    x[..., -1] = 1e37
+    w = torch.full((3, width), 200.0)
+    w[:, -1] = 1e-37
+    got = [t.to(DEV).requires_grad_(True) for t in (x, w)]
+    grads = torch.autograd.grad(causal_conv1d_fn(got[0], got[1], None, "silu"), got, dy.to(DEV))
+    ref = [t.double().requires_grad_(True) for t in (x, w)]
+    want = torch.autograd.grad(oracle.causal_conv1d(ref[0], ref[1], None, "silu")[0], ref, dy.double())
+    for name, g, r in zip(("x", "weight"), grads, want):
+        assert rel(g, r) <= 1e-4, (name, rel(g, r))
