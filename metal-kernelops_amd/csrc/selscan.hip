@@ -1584,12 +1584,13 @@ __global__ void __launch_bounds__(256) bwd_main(Geo g, Ptrs p) {
 
       if (UNI) {
         // The block's B/C rows, shared by the workgroup (the previous block's
-        // flush barrier orders this write after every read of the old rows).
+        // flush barrier orders this write after every read of the old rows), with zeros past the
+        // sequence: what lies there is the next row's, or nothing anyone wrote.
         for (int e = threadIdx.x; e < NS * HS; e += blockDim.x) {
           const int n = e / HS, i = e % HS;
           const int64_t src = (li.bg * NS + n) * g.length + qs + i;
-          rows_b[e] = p.bn[src];
-          rows_c[e] = p.cn[src];
+          rows_b[e] = i < nv ? p.bn[src] : 0.0f;
+          rows_c[e] = i < nv ? p.cn[src] : 0.0f;
         }
         __syncthreads();
       }
@@ -1614,6 +1615,13 @@ __global__ void __launch_bounds__(256) bwd_main(Geo g, Ptrs p) {
         } else {
           load_run_t<float, HS>(bn_p + n * static_cast<int64_t>(g.length), HS, (g.length % 4) == 0, bv);
           load_run_t<float, HS>(cn_p + n * static_cast<int64_t>(g.length), HS, (g.length % 4) == 0, cv);
+          if (nv < HS) {  // as above
+#pragma unroll
+            for (int i = 0; i < HS; ++i) {
+              bv[i] = i < nv ? bv[i] : 0.0f;
+              cv[i] = i < nv ? cv[i] : 0.0f;
+            }
+          }
         }
         const float an = arow[n];
         const float a2 = an * kLog2e;
