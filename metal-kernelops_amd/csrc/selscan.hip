@@ -2182,10 +2182,11 @@ static int launch_bwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_par
   g.lc = static_cast<int>((nblk + g.nchunks - 1) / g.nchunks) * HS;
   const unsigned gx = blocks_for(g.rows, 4 * kLaneChannels);
   // Taking the pre-gate output back from the rounded out adds that rounding to dz (2.35e-3 at
-  // 4 x 5120 x 4096 in bf16; problems that form the sum have 1.66e-3), so only the problems that fill the chip by themselves and are bound by vector
-  // issue do it, whole blocks of at least kLaneRows rows (4 x 5120 x 4096
-  // 1325 us against 1503 with the sum, 8 x 1536 x 2048 386 against 460).
-  const bool use_out = q.out != nullptr && g.rows >= kLaneRows;
+  // 4 x 5120 x 4096 in bf16, where forming the sum gives 1.66e-3), so only the problems that fill
+  // the chip by themselves and are bound by vector issue do it: whole blocks of aligned rows, at
+  // least kLaneRows of them (4 x 5120 x 4096 1325 us against 1503 with the sum, 8 x 1536 x 2048
+  // 386 against 460).
+  const bool use_out = q.out != nullptr && g.rows >= kLaneRows && g.vec;
   auto go = [&](auto tb, auto vbc) {
     using TB = decltype(tb);
     constexpr bool VBC = decltype(vbc)::value;

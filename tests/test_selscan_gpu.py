@@ -400,3 +400,28 @@ def test_ragged_rows_keep_apart(length):
         assert torch.equal(grads[k][:, 0], clean[1][k][:, 0]), k
     for k in ("A", "D", "delta_bias"):
         assert torch.equal(grads[k][:4], clean[1][k][:4]), k
+
+
+def _off_alignment(t):
+    """t's values one element past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    return flat[1:1 + t.numel()].view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("which", ["u", "z", "dy", "out"])
+def test_unaligned_rows_sum_the_pre_gate_output(which):
+    # dz comes from out / silu(z), with out's rounding, only where every row is aligned; any other
+    # call of 6144 rows sums C x over the states, and out makes no difference.
+    from metal_kernelops.scan import selscan_bwd_impl, selscan_fwd_impl
+    inputs, dy = _random_problem(2, 3072, 32, 16, 1, seed=47, act=torch.bfloat16)
+    dev = {k: v.to(DEV) for k, v in inputs.items()} | {"dy": dy.to(DEV)}
+    names = ("u", "dt", "A", "B", "C", "D", "z", "delta_bias")
+    dev["out"], states = selscan_fwd_impl(*(dev[k] for k in names), True)
+
+    def dz(t, out):
+        return selscan_bwd_impl(t["dy"], *(t[k] for k in names), True, states, out)[6]
+
+    summed = dz(dev, None)
+    assert not torch.equal(dz(dev, dev["out"]), summed)
+    moved = dev | {which: _off_alignment(dev[which])}
+    assert torch.equal(dz(moved, moved["out"]), summed)
