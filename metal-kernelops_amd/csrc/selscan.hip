@@ -657,6 +657,12 @@ __global__ void __launch_bounds__(256) fwd_replay(Geo g, Ptrs p) {
 // the recurrence, but a problem of few rows has no other work for the chip: one launch in
 // place of a layout pass, a summary, a chain and a replay.
 //
+// RESTART: what enters a block decays by e^{A sum of the block's steps} into the state leaving it,
+// and the block's own part is formed from a zero state beside the walk: one rounding of the decay
+// a block where the walk takes sixteen.  Without it the state drifts along the run, which shows in
+// dA of short problems (kRestartSteps); it costs 5-10% of a launch (5120 rows x 1003 steps, bf16, 49
+// -> 53 us; 384 x 1003 13.3 -> 14.0).
+//
 // Rows need no alignment and the length no whole blocks: elements past a row's end come from
 // the row after it or, past the last, read as zero (buffer range check), and only ever reach
 // the steps past the end, whose states nothing reads and whose outputs are not stored.
@@ -768,7 +774,7 @@ struct BcShare {
   }
 };
 
-template <class TU, class TB, bool VBC, int K>
+template <class TU, class TB, bool VBC, int K, bool RESTART>
 __global__ void __launch_bounds__((K > 4 ? K : 4) * kWave) __attribute__((amdgpu_waves_per_eu(K > 4 ? 4 : 5)))
 fwd_lane(Geo g, Ptrs p) {
   constexpr int kWaves = K > 4 ? K : 4;
@@ -843,10 +849,12 @@ fwd_lane(Geo g, Ptrs p) {
         float bv[HS];
         lds_row<HS>(brow, bv);
         wave_lds_sync();
+        float own = RESTART ? 0.0f : x;
         static_for<0, HS>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
-          x = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), x, row_newbcast<i>(du) * bv[i]);
+          own = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), own, row_newbcast<i>(du) * bv[i]);
         });
+        x = RESTART ? fmaf(fast_exp2(a2 * row16_sum(del)), x, own) : own;
         sum += del;
       };
       for (int k = b0; k < b1; k += 2) {
@@ -896,11 +904,16 @@ fwd_lane(Geo g, Ptrs p) {
     lds_row<HS>(brow, bv);
     lds_row<HS>(crow, cv);
     const float du = del * uu;
+    const float entering = x;
+    float own = 0.0f;  // what the block itself adds to the state leaving it
     static_for<0, HS>([&](auto ic) {
       constexpr int i = decltype(ic)::value;
-      x = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), x, row_newbcast<i>(du) * bv[i]);
+      const float a = fast_exp2(a2 * row_newbcast<i>(del)), add = row_newbcast<i>(du) * bv[i];
+      x = fmaf(a, x, add);
+      if constexpr (RESTART) own = fmaf(a, own, add);
       sw[i * kRow + n] = cv[i] * x;
     });
+    if constexpr (RESTART) x = fmaf(fast_exp2(a2 * row16_sum(del)), entering, own);
     wave_lds_sync();
     float s4[4];
 #pragma unroll
@@ -927,7 +940,11 @@ fwd_lane(Geo g, Ptrs p) {
 // into chunks (lane_bwd_chunks): bwd_map first walks every chunk but the first with the adjoint
 // alone, from a zero exit, which with the chunk's sum of steps gives its map from the adjoint
 // entering it on the right to the one leaving it on the left; bwd_lane composes the maps of
-// the chunks to the right of its own before its first block.
+// the chunks to the right of its own before its first block.  Unless FULL, the adjoint is carried
+// over a block as fwd_lane's RESTART carries the state: 16 rounded decays in a row are all that
+// ddelta and dA see, however long the chunk.  Carried as the product of its steps' decays, ddelta's
+// error against 64 bits was 1.75e-7 in the 2D scan of 384 channels, 28 x 28, now 1.03e-7, and dA's up
+// to 1.10 times what it is now; the backward takes 2-6% longer (5120 rows x 1003 steps 144 -> 149 us).
 // Per block:
 //   - lane (c, n) loads step t0 + n of its channel's delta, u, z, dout and out and forms that
 //     element's step, du, gy = dout silu(z) and the factor of dz;
@@ -948,8 +965,8 @@ fwd_lane(Geo g, Ptrs p) {
 //     the four rows of one register: 6 instructions per two steps, in a fixed order;
 //   - lane (c, n) then owns step t0 + n: it sums its row of the transpose and writes du,
 //     ddelta and dz.  The pre-gate output that dz needs comes from a transpose of C x summed
-//     over the states; with use_out it comes back as out / silu(z), except in a block where
-//     silu(z) is exactly zero somewhere;
+//     over the states; FULL takes it back as out / silu(z), except in a block where silu(z) is
+//     exactly zero somewhere;
 //   - the workgroup's 4 wavefronts add their dB/dC blocks in a fixed order and write one
 //     partial per 16 channels (per 4 channels when a group is not a multiple of 16 wide).
 // It is bound by vector issue.  B and C pass through the transpose buffer, so a workgroup's LDS
@@ -1052,10 +1069,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
     float cv[HS];
     lds_row<HS>(&sbc[wave][n][0], cv);
     wave_lds_sync();
+    // the block's own part from a zero adjoint; what enters it decays by the block's sum of steps
+    float own = 0.0f;
     static_for<0, HS>([&](auto jc) {
       constexpr int i = HS - 1 - decltype(jc)::value;
-      h = fast_exp2(row_bcast<i>(del) * a2) * fmaf(row_bcast<i>(gy), cv[i], h);
+      own = fast_exp2(row_bcast<i>(del) * a2) * fmaf(row_bcast<i>(gy), cv[i], own);
     });
+    h = fmaf(fast_exp2(a2 * row16_sum(del)), h, own);
     sum += del;
   };
   for (int k = b1 - 1; k >= b0; k -= 2) {
@@ -1070,9 +1090,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
   }
 }
 
-template <class TU, class TB, bool VBC>
+template <class TU, class TB, bool VBC, bool FULL>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VBC ? 4 : 3)))
-bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
+bwd_lane(Geo g, Ptrs p, int cpb) {
   // per wavefront: the transposes of the pairs (h B, a x h); in blocks that need it, the
   // first terms first transpose C x; the workgroup's dB/dC blocks reuse the buffers
   __shared__ __align__(16) float lds[4][kTrFloats];
@@ -1090,7 +1110,7 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
   const float bias = p.bias ? p.bias[d] : 0.0f;
   const float Dd = p.D ? p.D[d] : 0.0f;
   const bool has_z = p.z != nullptr;
-  const bool has_out = use_out;
+  const bool has_out = FULL && p.out != nullptr;
   const int L = static_cast<int>(g.length);
   float* tr = lds[wave];
   // The wavefront's rows of the per-element arrays and its group's of B and C as buffers; this
@@ -1218,19 +1238,23 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
       recompute(std::false_type{});
     }
     // ---- reverse walk
-    float dA0, dA1;  // the block's dA in two chains (even, odd steps)
+    // the block's dA, step i in chain i mod kChains (four take 1.5% off dA's error at 190-1003
+    // steps and no time; FULL has no register for them)
+    constexpr int kChains = FULL ? 2 : 4;
+    float dAc[kChains];
     float sbc[HS / 2];  // dB/dC of step pairs summed over the wavefront's 4 channels (see below)
     float rodd = 0.0f;  // the odd step's half-summed register, waiting for its even partner
+    const float entering = carry;
+    float own = 0.0f;  // what the block itself adds to the adjoint leaving it
     static_for<0, HS>([&](auto jc) {
       constexpr int i = HS - 1 - decltype(jc)::value;
       const float h = fmac_row<i, i == HS - 1>(carry, gy, cv[i]);
       const float hc = ah[i] * h;
+      if constexpr (!FULL) own = ah[i] * (i == HS - 1 ? row_bcast<i>(gy) * cv[i] : fmac_row<i>(own, gy, cv[i]));
       const float pr = hc * (i > 0 ? xh[i > 0 ? i - 1 : 0] : x0);
       *reinterpret_cast<float2*>(tr + i * kTrPitch + 2 * tw) = make_float2(h * bv[i], pr);
-      if constexpr (i == HS - 1) dA1 = row_bcast<i>(del) * pr;
-      else if constexpr (i == HS - 2) dA0 = row_bcast<i>(del) * pr;
-      else if constexpr (i % 2 == 0) dA0 = fmac_row<i>(dA0, del, pr);
-      else dA1 = fmac_row<i>(dA1, del, pr);
+      if constexpr (i >= HS - kChains) dAc[i % kChains] = row_bcast<i>(del) * pr;
+      else dAc[i % kChains] = fmac_row<i>(dAc[i % kChains], del, pr);
       // dB and dC terms of step i, h du_i and gy_i x_i: rows c0 + c2 and c1 + c3 of each
       // (a swap of the wavefront's halves), dB in rows 0-1 and dC in rows 2-3 ...
       const float pb = row_bcast<i>(du) * h, pc = row_bcast<i>(gy) * xh[i];
@@ -1246,10 +1270,13 @@ bwd_lane(Geo g, Ptrs p, int cpb, bool use_out) {
       }
       carry = hc;
     });
+    if constexpr (!FULL) carry = fmaf(fast_exp2(a2 * row16_sum(del)), entering, own);
     // summed over 8 blocks at a time: a long chunk's rounding grows with the terms added in a
     // row (dA's error against 64 bits: 4 x 5120 x 4096 bf16 3.62e-7 -> 2.48e-7, 3 x 4096 x 2055 fp32
     // 3.02e-7 -> 2.37e-7; the backward's time is the same)
-    dA_run += dA0 + dA1;
+    float dA_blk = dAc[0] + dAc[1];
+    if constexpr (!FULL) dA_blk += dAc[2] + dAc[3];
+    dA_run += dA_blk;
     if (k % 8 == 0) {
       dA_acc += dA_run;
       dA_run = 0.0f;
@@ -1929,23 +1956,34 @@ static int lane_chunks(const Geo& g) {
   return quads <= 384 && nblk >= 32 ? 16 : 4;
 }
 
-// Time chunks of the lane-per-state backward: the smallest power of two that gives each of 1024
-// SIMDs 3 wavefronts, with at least four blocks each.  (bwd_lane holds four a SIMD since its LDS
-// and registers were cut; the figures are from before, and the line was not moved.)
-// A chunk costs its bwd_map and its own dA / dD / ddelta_bias partials.  us a backward with
-// 1 / 2 / 4 / 8 / 32 chunks, bf16: 5120 rows x 1024 steps 153 / 131 / 116 / 117 / 149, 1536 x 2048
-// 210 / 141 / 101 / 78 / 84, 384 x 3136 309 / 199 / 110 / 67 / 48, 8 x 1536 x 2048 413 / 436.
+// Time chunks of the lane-per-state backward: one where the rows give each of the 1024 SIMDs 3
+// wavefronts, else the smallest power of two up to 64 that gives them 4 (as many as bwd_lane's LDS
+// and registers allow), with at least four blocks each.  A chunk costs its bwd_map and its own dA /
+// dD / ddelta_bias partials.  us a backward, bf16, splitting up to 3 wavefronts a SIMD / 4 / 6:
+// 768 rows x 4096 steps 90 / 88 / 86, 1536 x 4096 167 / 159 / 163, 3072 x 2048 171 / 164 / 169,
+// 3072 x 8192 609 / 584 / 592; 12288 x 1024, which has 3 from its rows, 234 in one chunk, 257 in two.
 static int lane_bwd_chunks(const Geo& g) {
   const int64_t quads = g.rows / kLaneChannels;
   const int64_t nblk = (g.length + HS - 1) / HS;
   int64_t k = 1;
-  // Steps taken as they are carry no softplus rounding, and ddelta then shows that of the decays'
-  // products along a chunk (2.1e-7 of it over 112 steps, 1.75e-7 over 64): chunks half as long.
-  const int64_t slots = g.softplus ? 3072 : 6144;
-  while (k < slots / 96 && quads * k < slots && nblk >= 8 * k) k <<= 1;
+  if (quads < 3072)
+    while (k < 64 && quads * k < 4096 && nblk >= 8 * k) k <<= 1;
   const int64_t per = (nblk + k - 1) / k;
   return static_cast<int>((nblk + per - 1) / per);
 }
+
+// Problems that fill the chip by themselves, in whole blocks of aligned rows: bound by vector issue
+// alone, they carry state and adjoint through the whole sequence as the products of the steps'
+// decays, and the backward takes the pre-gate output back from the rounded out, which adds that
+// rounding to dz (2.35e-3 at 4 x 5120 x 4096 in bf16, where the sum over the states gives 1.66e-3;
+// 1325 us against 1503 with the sum, 8 x 1536 x 2048 386 against 460).
+static bool full_walk(const Geo& g) { return g.rows >= kLaneRows && g.vec && g.length % HS == 0; }
+
+// Longest sequence whose forward restarts at every block.  dA's error without the restart over its
+// error on the lane-per-channel mapping, fp32, the worst of 256 to 8192 rows: 1.02 at 200 and 320
+// steps, 1.01 at 780 and 1003, 1.006 at 1200, 0.97 at 1600, 0.96 at 2500 (its sums over more blocks
+// are the better ones); with it 1.00 at most.  The other results are below 1 either way.
+constexpr int64_t kRestartSteps = 96 * HS;
 
 // The backward's too.  It indexes the per-row arrays (u, delta, z, dout, out, du, ddelta, dz,
 // the saved states) and B/C with 32-bit lane offsets from a 64-bit base, so each of them must
@@ -2116,25 +2154,28 @@ static bool chain_by_wave(const Geo& g) {
 }
 
 
-template <class TU, class TB, bool VBC>
-static void launch_fwd_lane_t(const Geo& g, int k, const Ptrs& q, hipStream_t s) {
+template <class TU, class TB, bool VBC, bool RESTART>
+static void launch_fwd_lane_t(const Geo& g, const Ptrs& q, hipStream_t s) {
+  const int k = lane_chunks(g);
   const int64_t quads = g.rows / kLaneChannels;
   if (k == 1)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1><<<blocks_for(quads, 4), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, RESTART><<<blocks_for(quads, 4), 256, 0, s>>>(g, q));
   else if (k == 4)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4><<<blocks_for(quads, 1), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4, RESTART><<<blocks_for(quads, 1), 256, 0, s>>>(g, q));
   else
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16><<<blocks_for(quads, 1), 1024, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16, RESTART><<<blocks_for(quads, 1), 1024, 0, s>>>(g, q));
 }
 
 template <class TU>
 static int launch_fwd_lane(const Plan& pl, const Ptrs& q, hipStream_t s) {
   const Geo& g = pl.g;
-  const int k = lane_chunks(g);
+  const bool restart = !(pl.vbc && full_walk(g)) && g.length <= kRestartSteps;
   auto go = [&](auto tb) {
     using TB = decltype(tb);
-    if (pl.vbc) launch_fwd_lane_t<TU, TB, true>(g, k, q, s);
-    else launch_fwd_lane_t<TU, TB, false>(g, k, q, s);
+    if (pl.vbc && restart) launch_fwd_lane_t<TU, TB, true, true>(g, q, s);
+    else if (pl.vbc) launch_fwd_lane_t<TU, TB, true, false>(g, q, s);
+    else if (restart) launch_fwd_lane_t<TU, TB, false, true>(g, q, s);
+    else launch_fwd_lane_t<TU, TB, false, false>(g, q, s);
   };
   if (g.bc_dtype == MKO_BF16) go(bf16{});
   else if (g.bc_dtype == MKO_F16) go(_Float16{});
@@ -2181,22 +2222,18 @@ static int launch_bwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_par
   const int64_t nblk = (g.length + HS - 1) / HS;
   g.lc = static_cast<int>((nblk + g.nchunks - 1) / g.nchunks) * HS;
   const unsigned gx = blocks_for(g.rows, 4 * kLaneChannels);
-  // Taking the pre-gate output back from the rounded out adds that rounding to dz (2.35e-3 at
-  // 4 x 5120 x 4096 in bf16, where forming the sum gives 1.66e-3), so only the problems that fill
-  // the chip by themselves and are bound by vector issue do it: whole blocks of aligned rows, at
-  // least kLaneRows of them (4 x 5120 x 4096 1325 us against 1503 with the sum, 8 x 1536 x 2048
-  // 386 against 460).
-  const bool use_out = q.out != nullptr && g.rows >= kLaneRows && g.vec;
-  auto go = [&](auto tb, auto vbc) {
+  auto go = [&](auto tb, auto vbc, auto full) {
     using TB = decltype(tb);
-    constexpr bool VBC = decltype(vbc)::value;
+    constexpr bool VBC = decltype(vbc)::value, FULL = decltype(full)::value;
     if (g.nchunks > 1)
       MKO_TIMED("selscan_bwd_map", s, bwd_map<TU, TB, VBC><<<dim3(gx, g.nchunks - 1), 256, 0, s>>>(g, q));
-    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, TB, VBC><<<dim3(gx, g.nchunks), 256, 0, s>>>(g, q, pl.cpb, VBC && use_out));
+    MKO_TIMED("selscan_bwd_lane", s, bwd_lane<TU, TB, VBC, FULL><<<dim3(gx, g.nchunks), 256, 0, s>>>(g, q, pl.cpb));
   };
+  const bool vbc = pl.vbc && g.length % HS == 0;
   auto go_b = [&](auto tb) {
-    if (pl.vbc && g.length % HS == 0) go(tb, std::true_type{});
-    else go(tb, std::false_type{});
+    if (vbc && full_walk(g)) go(tb, std::true_type{}, std::true_type{});
+    else if (vbc) go(tb, std::true_type{}, std::false_type{});
+    else go(tb, std::false_type{}, std::false_type{});
   };
   if (g.bc_dtype == MKO_BF16) go_b(bf16{});
   else if (g.bc_dtype == MKO_F16) go_b(_Float16{});
