@@ -660,8 +660,9 @@ __global__ void __launch_bounds__(256) fwd_replay(Geo g, Ptrs p) {
 // RESTART: what enters a block decays by e^{A sum of the block's steps} into the state leaving it,
 // and the block's own part is formed from a zero state beside the walk: one rounding of the decay
 // a block where the walk takes sixteen.  Without it the state drifts along the run, which shows in
-// dA of short problems (kRestartSteps); it costs 5-10% of a launch (5120 rows x 1003 steps, bf16, 49
-// -> 53 us; 384 x 1003 13.3 -> 14.0).
+// dA of short problems (kRestartSteps); it costs 5-10% of a launch (5120 rows x 256 steps, bf16,
+// 14.9 -> 16.2 us).  The maps of a run's entering state alone, which need no second chain, restart
+// up to kMapRestartSteps (5120 x 1003 steps 43.4 -> 44.9 us).
 //
 // Rows need no alignment and the length no whole blocks: elements past a row's end come from
 // the row after it or, past the last, read as zero (buffer range check), and only ever reach
@@ -682,6 +683,14 @@ __device__ __forceinline__ float row_newbcast(float v) {
 }
 
 constexpr int kLaneChannels = 4;  // channels per wavefront in the lane-per-state kernels
+
+// Longest sequences whose forward restarts at every block, and whose runs' maps do.  dA's error over
+// that of the lane-per-channel mapping, fp32, the worst of 256 to 8192 rows, with no restart / with
+// the maps': 1.03 / 1.02 at 200, 320 and 461 steps, 1.01 / 1.005 at 700 to 1200, 0.97 at 1600, 0.96 at
+// 2500 (its sums over more blocks are the better ones); with both at most 1.00.  The other results
+// are below 1 without.
+constexpr int64_t kRestartSteps = 40 * HS;
+constexpr int64_t kMapRestartSteps = 96 * HS;
 
 // One 16-step block of B and C staged through LDS for a wavefront of the lane-per-state
 // kernels, whose 4 channels share one (batch, group).  Rows are kBcRow floats: 16-byte
@@ -836,6 +845,7 @@ fwd_lane(Geo g, Ptrs p) {
   if constexpr (K > 1) {
     // ---- the run's map, from a zero entry; the last run's is not needed
     constexpr auto kMap = std::false_type{};
+    const bool map_restart = g.length <= kMapRestartSteps;
     if (kc < K - 1 && b0 < b1) {
       float sum = 0.0f;
       load(b0, ra, kMap);
@@ -849,12 +859,13 @@ fwd_lane(Geo g, Ptrs p) {
         float bv[HS];
         lds_row<HS>(brow, bv);
         wave_lds_sync();
-        float own = RESTART ? 0.0f : x;
+        float own = map_restart ? 0.0f : x;
         static_for<0, HS>([&](auto ic) {
           constexpr int i = decltype(ic)::value;
           own = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), own, row_newbcast<i>(du) * bv[i]);
         });
-        x = RESTART ? fmaf(fast_exp2(a2 * row16_sum(del)), x, own) : own;
+        if (map_restart) x = fmaf(fast_exp2(a2 * row16_sum(del)), x, own);
+        else x = own;
         sum += del;
       };
       for (int k = b0; k < b1; k += 2) {
@@ -1978,12 +1989,6 @@ static int lane_bwd_chunks(const Geo& g) {
 // rounding to dz (2.35e-3 at 4 x 5120 x 4096 in bf16, where the sum over the states gives 1.66e-3;
 // 1325 us against 1503 with the sum, 8 x 1536 x 2048 386 against 460).
 static bool full_walk(const Geo& g) { return g.rows >= kLaneRows && g.vec && g.length % HS == 0; }
-
-// Longest sequence whose forward restarts at every block.  dA's error without the restart over its
-// error on the lane-per-channel mapping, fp32, the worst of 256 to 8192 rows: 1.02 at 200 and 320
-// steps, 1.01 at 780 and 1003, 1.006 at 1200, 0.97 at 1600, 0.96 at 2500 (its sums over more blocks
-// are the better ones); with it 1.00 at most.  The other results are below 1 either way.
-constexpr int64_t kRestartSteps = 96 * HS;
 
 // The backward's too.  It indexes the per-row arrays (u, delta, z, dout, out, du, ddelta, dz,
 // the saved states) and B/C with 32-bit lane offsets from a 64-bit base, so each of them must
