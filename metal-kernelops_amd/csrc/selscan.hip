@@ -24,6 +24,7 @@
 // Per-step inputs of the state-inner loops (one lane, all states, one step at a
 // time) are staged through LDS so the step loop is a real loop and B_t/C_t are
 // fetched one step at a time.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -656,6 +657,10 @@ __global__ void __launch_bounds__(256) fwd_replay(Geo g, Ptrs p) {
 // its own, and walks its run again from that entering state.  The runs cost a second pass over
 // the recurrence, but a problem of few rows has no other work for the chip: one launch in
 // place of a layout pass, a summary, a chain and a replay.
+// Sequences so long that 16 runs still leave SIMDs idle are cut into time chunks instead
+// (blockIdx.y, K = 1): fwd_map forms every chunk's map but the last's, and each wavefront composes
+// those before its chunk.  us a forward, bf16, with 16 runs / in chunks: 64 rows x 4096 steps
+// 37 / 15, 64 x 131072 1061 / 105 (lane per channel 146), 384 x 16384 145 / 70 (135).
 //
 // RESTART: what enters a block decays by e^{A sum of the block's steps} into the state leaving it,
 // and the block's own part is formed from a zero state beside the walk: one rounding of the decay
@@ -783,6 +788,74 @@ struct BcShare {
   }
 };
 
+// One chunk's map of the state: from a zero state entering it, the state that leaves it, and its
+// sum of steps.  The last chunk's is never needed, so every block here is whole.
+template <class TU, class TB, bool VBC>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) fwd_map(Geo g, Ptrs p) {
+  __shared__ __align__(16) float sbc[4][HS][kBcRow];
+  const int wave = uniform(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63, cl = lane >> 4, n = lane & 15;
+  int64_t row0 = (static_cast<int64_t>(blockIdx.x) * 4 + wave) * kLaneChannels;
+  const bool active = row0 < g.rows;
+  if (!active) row0 = g.rows - kLaneChannels;
+  const int64_t bg = uniform(static_cast<int>(row0 / g.dg));
+  const int64_t d = row0 % g.dim + cl;
+  const int N = static_cast<int>(g.dstate);
+  const float a2 = n < N ? p.A[d * N + n] * kLog2e : 0.0f;
+  const float bias = p.bias ? p.bias[d] : 0.0f;
+  const int L = static_cast<int>(g.length);
+  const int c = blockIdx.y, per = g.lc / HS;
+  const int b0 = c * per, b1 = b0 + per;
+  constexpr uint32_t kU = sizeof(TU);
+  const uint32_t rows = kLaneChannels * static_cast<uint32_t>(L);
+  const auto rdl = raw_buffer(static_cast<const float*>(p.delta) + row0 * L, rows * 4);
+  const auto ru = raw_buffer(static_cast<const TU*>(p.u) + row0 * L, rows * kU);
+  const auto rB = raw_buffer(static_cast<const TB*>(p.B) + bg * N * L, N * static_cast<uint32_t>(L) * sizeof(TB));
+  const uint32_t eoff = static_cast<uint32_t>(cl) * L + n;
+  const auto share = BcShare<TB, VBC>::at(lane, N, L, &sbc[wave][0][0]);
+  struct In {
+    uint32_t dl, u;
+    BcShare<TB, VBC> b;
+  };
+  auto load = [&](int k, In& in) {
+    const uint32_t t0 = static_cast<uint32_t>(k < b1 ? k : b1 - 1) * HS;
+    in.dl = buffer_word<float>(rdl, (eoff + t0) * 4);
+    in.u = buffer_word<TU>(ru, (eoff + t0) * kU);
+    in.b.load(rB, share, t0);
+  };
+  In ra, rb;
+  load(b0, ra);
+  load(b0 + 1, rb);
+  float x = 0.0f, sum = 0.0f;
+  auto block = [&](int k, In& in) {
+    const float del = step_of(g, __uint_as_float(in.dl), bias);
+    const float du = del * word_f32<TU>(in.u);
+    in.b.put(share, 0);
+    load(k + 2, in);
+    wave_lds_sync();
+    float bv[HS];
+    lds_row<HS>(&sbc[wave][n][0], bv);
+    wave_lds_sync();
+    float own = 0.0f;
+    static_for<0, HS>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      own = fmaf(fast_exp2(a2 * row_newbcast<i>(del)), own, row_newbcast<i>(du) * bv[i]);
+    });
+    x = fmaf(fast_exp2(a2 * row16_sum(del)), x, own);
+    sum += del;
+  };
+  for (int k = b0; k < b1; k += 2) {
+    block(k, ra);
+    if (k + 1 < b1) block(k + 1, rb);
+  }
+  sum = row16_sum(sum);
+  if (active) {
+    const int64_t o = c * g.rows + row0 + cl;
+    p.drive[o * HS + n] = x;
+    if (n == 0) p.sumd[o] = sum;
+  }
+}
+
 template <class TU, class TB, bool VBC, int K, bool RESTART>
 __global__ void __launch_bounds__((K > 4 ? K : 4) * kWave) __attribute__((amdgpu_waves_per_eu(K > 4 ? 4 : 5)))
 fwd_lane(Geo g, Ptrs p) {
@@ -808,8 +881,9 @@ fwd_lane(Geo g, Ptrs p) {
   const bool has_z = p.z != nullptr;
   const int L = static_cast<int>(g.length);
   const int nblk = (L + HS - 1) / HS;
-  const int per = (nblk + K - 1) / K;
-  const int b0 = kc * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+  const int per = K > 1 ? (nblk + K - 1) / K : (RESTART ? nblk : g.lc / HS);
+  const int b0 = K > 1 ? kc * per : (RESTART ? 0 : static_cast<int>(blockIdx.y) * per);
+  const int b1 = b0 + per < nblk ? b0 + per : nblk;
   // the wavefront's rows of the per-element arrays, and its group's of B and C
   constexpr uint32_t kU = sizeof(TU), kB = sizeof(TB);
   const uint32_t rows = kLaneChannels * static_cast<uint32_t>(L);
@@ -884,6 +958,22 @@ fwd_lane(Geo g, Ptrs p) {
       x = fmaf(m[0], x, m[1]);
     }
     __syncthreads();  // the transposes take the buffers
+  } else if constexpr (!RESTART) {
+    // the maps of the chunks before this one (fwd_map's; none with RESTART), fetched eight at a time (clamped: every
+    // load is issued)
+    const int ch = blockIdx.y;
+    for (int c0 = 0; c0 < ch; c0 += 8) {
+      float e[8], m[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int64_t o = (c0 + q < ch ? c0 + q : ch - 1) * g.rows + row0 + cl;
+        e[q] = p.sumd[o];
+        m[q] = p.drive[o * HS + n];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (c0 + q < ch) x = fmaf(fast_exp2(a2 * e[q]), x, m[q]);
+    }
   }
 
   // ---- outputs and saved states
@@ -1939,6 +2029,8 @@ struct Plan {
   int cpb, lchunks;
   int64_t lncb;
   size_t loff_pbc, loff_dap, loff_ddp, loff_dbp, loff_drive, loff_sumd;
+  int fchunks;  // fwd_lane's time chunks; their maps, from offset 0 of the forward's workspace
+  size_t foff_sumd;
   size_t fwd_bytes, bwd_bytes;
 };
 
@@ -1967,20 +2059,29 @@ static int lane_chunks(const Geo& g) {
   return quads <= 384 && nblk >= 32 ? 16 : 4;
 }
 
-// Time chunks of the lane-per-state backward: one where the rows give each of the 1024 SIMDs 3
-// wavefronts, else the smallest power of two up to 64 that gives them 4 (as many as bwd_lane's LDS
-// and registers allow), with at least four blocks each.  A chunk costs its bwd_map and its own dA /
-// dD / ddelta_bias partials.  us a backward, bf16, splitting up to 3 wavefronts a SIMD / 4 / 6:
-// 768 rows x 4096 steps 90 / 88 / 86, 1536 x 4096 167 / 159 / 163, 3072 x 2048 171 / 164 / 169,
-// 3072 x 8192 609 / 584 / 592; 12288 x 1024, which has 3 from its rows, 234 in one chunk, 257 in two.
-static int lane_bwd_chunks(const Geo& g) {
+// Time chunks of the lane-per-state mapping: one where the rows give each of the 1024 SIMDs 3
+// wavefronts, else the smallest power of two that gives them 4 (as many as bwd_lane's LDS and
+// registers allow), with at least four blocks each, and past 64 chunks at least half as many blocks
+// as there are chunks, since every chunk composes the maps of those beside it.  A chunk costs its
+// map and, in the backward, its own dA / dD / ddelta_bias partials.  us a backward, bf16, splitting
+// up to 3 wavefronts a SIMD / 4 / 6: 768 rows x 4096 steps 90 / 88 / 86, 1536 x 4096 167 / 159 / 163,
+// 3072 x 2048 171 / 164 / 169, 3072 x 8192 609 / 584 / 592; 12288 x 1024, which has 3 from its rows,
+// 234 in one chunk, 257 in two.  At 131072 steps with at most 64 chunks / as here: 4 rows 267 / 123,
+// 64 rows 314 / 247, 256 rows 894 / 808.
+static int lane_time_chunks(const Geo& g) {
   const int64_t quads = g.rows / kLaneChannels;
   const int64_t nblk = (g.length + HS - 1) / HS;
   int64_t k = 1;
   if (quads < 3072)
-    while (k < 64 && quads * k < 4096 && nblk >= 8 * k) k <<= 1;
+    while (quads * k < 4096 && nblk >= 8 * k && (k < 64 || nblk >= k * k / 2)) k <<= 1;
   const int64_t per = (nblk + k - 1) / k;
   return static_cast<int>((nblk + per - 1) / per);
+}
+
+// The forward takes them where they are more than its 16 runs (of one launch and one map less).
+static int lane_fwd_chunks(const Geo& g) {
+  const int k = lane_time_chunks(g);
+  return k > 16 ? k : 1;
 }
 
 // Problems that fill the chip by themselves, in whole blocks of aligned rows: bound by vector issue
@@ -2080,6 +2181,13 @@ static int make_plan(const mko_selscan_params* p, Plan* pl) {
   pl->off_drive = o; o = align_up(o + rk * g.dstate * 4);
   pl->off_sumd = o; o = align_up(o + rk * 4);
   pl->fwd_bytes = o;
+  pl->fchunks = 1;
+  if (lane_shape(g, pl->ns) && g.length > 0) {
+    pl->fchunks = lane_fwd_chunks(g);
+    const size_t maps = static_cast<size_t>(g.rows) * (pl->fchunks - 1);
+    pl->foff_sumd = align_up(maps * HS * 4);
+    pl->fwd_bytes = std::max(pl->fwd_bytes, align_up(pl->foff_sumd + maps * 4));
+  }
   // backward workspace (extends the forward layout: bt/ct are used by both)
   pl->off_bn = o; o = align_up(o + (bgl * ns + HS) * 4);  // + one row tail: blocks read HS steps
   pl->off_cn = o; o = align_up(o + (bgl * ns + HS) * 4);
@@ -2093,7 +2201,7 @@ static int make_plan(const mko_selscan_params* p, Plan* pl) {
   pl->cpb = (g.dg % 16) == 0 ? 16 : 4;
   pl->lncb = g.dg / pl->cpb;
   if (lane_bwd_shape(g, pl->ns)) {
-    pl->lchunks = g.length > 0 ? lane_bwd_chunks(g) : 1;
+    pl->lchunks = g.length > 0 ? lane_time_chunks(g) : 1;
     const size_t rch = static_cast<size_t>(g.rows) * pl->lchunks;
     size_t q = 0;
     pl->loff_pbc = q; q = align_up(q + static_cast<size_t>(g.batch * g.ngroups) * pl->lncb * g.length * 16 * 2 * 4);
@@ -2161,20 +2269,32 @@ static bool chain_by_wave(const Geo& g) {
 
 template <class TU, class TB, bool VBC, bool RESTART>
 static void launch_fwd_lane_t(const Geo& g, const Ptrs& q, hipStream_t s) {
-  const int k = lane_chunks(g);
+  const int k = g.nchunks > 1 ? 1 : lane_chunks(g);
   const int64_t quads = g.rows / kLaneChannels;
+  const dim3 grid(blocks_for(quads, k == 1 ? 4 : 1), g.nchunks);
+  if constexpr (!RESTART) {
+    if (g.nchunks > 1)
+      MKO_TIMED("selscan_fwd_map", s, fwd_map<TU, TB, VBC><<<dim3(grid.x, g.nchunks - 1), 256, 0, s>>>(g, q));
+  }
   if (k == 1)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, RESTART><<<blocks_for(quads, 4), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, RESTART><<<grid, 256, 0, s>>>(g, q));
   else if (k == 4)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4, RESTART><<<blocks_for(quads, 1), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4, RESTART><<<grid, 256, 0, s>>>(g, q));
   else
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16, RESTART><<<blocks_for(quads, 1), 1024, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16, RESTART><<<grid, 1024, 0, s>>>(g, q));
 }
 
 template <class TU>
-static int launch_fwd_lane(const Plan& pl, const Ptrs& q, hipStream_t s) {
-  const Geo& g = pl.g;
-  const bool restart = !(pl.vbc && full_walk(g)) && g.length <= kRestartSteps;
+static int launch_fwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_params* p, hipStream_t s) {
+  Geo g = pl.g;
+  g.nchunks = pl.fchunks;
+  const int64_t nblk = (g.length + HS - 1) / HS;
+  g.lc = static_cast<int>((nblk + g.nchunks - 1) / g.nchunks) * HS;
+  Ptrs q = q0;
+  q.drive = static_cast<float*>(p->workspace);
+  q.sumd = reinterpret_cast<float*>(static_cast<char*>(p->workspace) + pl.foff_sumd);
+  // chunks are of sequences past kRestartSteps (128 blocks and more)
+  const bool restart = g.nchunks == 1 && !(pl.vbc && full_walk(g)) && g.length <= kRestartSteps;
   auto go = [&](auto tb) {
     using TB = decltype(tb);
     if (pl.vbc && restart) launch_fwd_lane_t<TU, TB, true, true>(g, q, s);
@@ -2345,9 +2465,9 @@ extern "C" int mko_selscan_fwd(const mko_selscan_params* p, void* stream) {
   Ptrs q = make_ptrs(p, pl);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (pl.lane) {
-    if (p->u_dtype == MKO_BF16) return launch_fwd_lane<bf16>(pl, q, s);
-    if (p->u_dtype == MKO_F16) return launch_fwd_lane<_Float16>(pl, q, s);
-    return launch_fwd_lane<float>(pl, q, s);
+    if (p->u_dtype == MKO_BF16) return launch_fwd_lane<bf16>(pl, q, p, s);
+    if (p->u_dtype == MKO_F16) return launch_fwd_lane<_Float16>(pl, q, p, s);
+    return launch_fwd_lane<float>(pl, q, p, s);
   }
   return dispatch_types(pl, p->u_dtype, p->delta_dtype, [&](auto tag) {
     using TU = decltype(tag);

@@ -447,3 +447,49 @@ def test_rounded_decays_do_not_pile_up(dim, length, dstate):
     _, want = _ref(inputs, dy, False)
     e = record(f"decays {dim}x{length}", "ddt", norm_rel(grads["dt"], want["dt"]), 1.5e-7)
     assert e <= 1.5e-7, f"{e:.3e}"
+
+
+# Sequences long for their rows are cut into time chunks in both directions: the shortest that are
+# (128 blocks of 16 steps, 32 chunks of 4), a ragged end with padded states, a short last chunk,
+# 16-bit rows off 16 bytes, and more than 64 chunks (half as many blocks to a chunk as chunks).
+CHUNK_SHAPES = [(1, 4, 2048, 16, 1), (1, 8, 2050, 5, 2), (2, 12, 3100, 16, 3), (1, 16, 4099, 9, 1), (1, 4, 32771, 16, 1)]
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16], ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("shape", CHUNK_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_long_sequences_in_time_chunks(shape, act):
+    if shape[2] > 10000 and act != torch.float32:
+        pytest.skip("one type at the longest: its oracle takes seconds")
+    inputs, dy = _random_problem(*shape, seed=sum(shape) + 3, act=act)
+    assert {"selscan_fwd_map", "selscan_fwd_lane"} <= _forward_kernels(inputs, True)
+    assert {"selscan_bwd_map", "selscan_bwd_lane"} <= _backward_kernels(inputs, dy)
+    _compare(inputs, dy, True, "chunks " + "x".join(map(str, shape)) + f" {act}")
+
+
+def test_long_few_rows_keep_the_chip_busy():
+    # 64 rows of 65536 steps: with time cut into 16 runs (forward) and 32 chunks (backward) most of
+    # the chip idled for 530 and 300 us.  Bars between those and the times in chunks (60 and 140 us).
+    def timed(fn):
+        fn()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(4):
+                fn()
+        times = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b) * 250)
+        return sorted(times)[2]
+
+    from metal_kernelops.scan import selscan_bwd_impl, selscan_fwd_impl
+    inputs, dy = _random_problem(1, 64, 65536, 16, 1, seed=5, act=torch.bfloat16)
+    args = [inputs[k].to(DEV) for k in NAMES]
+    dy = dy.to(DEV)
+    _, states = selscan_fwd_impl(*args, True)
+    assert timed(lambda: selscan_fwd_impl(*args, True)) < 300
+    assert timed(lambda: selscan_bwd_impl(dy, *args, True, states)) < 230
