@@ -856,9 +856,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) f
   }
 }
 
-template <class TU, class TB, bool VBC, int K, bool RESTART>
+// CHUNKS is a mode of its own: the loop over the maps costs the others registers (6144 rows x 6272
+// steps fp32 347 -> 400 us).
+enum Walk { WHOLE, RESTARTS, CHUNKS };
+
+template <class TU, class TB, bool VBC, int K, Walk WALK>
 __global__ void __launch_bounds__((K > 4 ? K : 4) * kWave) __attribute__((amdgpu_waves_per_eu(K > 4 ? 4 : 5)))
 fwd_lane(Geo g, Ptrs p) {
+  constexpr bool RESTART = WALK == RESTARTS;
+  static_assert(WALK != CHUNKS || K == 1, "chunks in place of runs");
   constexpr int kWaves = K > 4 ? K : 4;
   constexpr int kRow = HS + 1;   // a step's 16 states, padded so the transposed reads miss no bank
   constexpr int kCS = HS * kRow; // one channel's [step][state] block (272 floats: 16 banks apart)
@@ -881,8 +887,8 @@ fwd_lane(Geo g, Ptrs p) {
   const bool has_z = p.z != nullptr;
   const int L = static_cast<int>(g.length);
   const int nblk = (L + HS - 1) / HS;
-  const int per = K > 1 ? (nblk + K - 1) / K : (RESTART ? nblk : g.lc / HS);
-  const int b0 = K > 1 ? kc * per : (RESTART ? 0 : static_cast<int>(blockIdx.y) * per);
+  const int per = WALK == CHUNKS ? g.lc / HS : (nblk + K - 1) / K;
+  const int b0 = (WALK == CHUNKS ? static_cast<int>(blockIdx.y) : kc) * per;
   const int b1 = b0 + per < nblk ? b0 + per : nblk;
   // the wavefront's rows of the per-element arrays, and its group's of B and C
   constexpr uint32_t kU = sizeof(TU), kB = sizeof(TB);
@@ -958,8 +964,9 @@ fwd_lane(Geo g, Ptrs p) {
       x = fmaf(m[0], x, m[1]);
     }
     __syncthreads();  // the transposes take the buffers
-  } else if constexpr (!RESTART) {
-    // the maps of the chunks before this one (fwd_map's; none with RESTART), fetched eight at a time (clamped: every
+  }
+  if constexpr (WALK == CHUNKS) {
+    // the maps of the chunks before this one (fwd_map's), fetched eight at a time (clamped: every
     // load is issued)
     const int ch = blockIdx.y;
     for (int c0 = 0; c0 < ch; c0 += 8) {
@@ -2059,20 +2066,20 @@ static int lane_chunks(const Geo& g) {
   return quads <= 384 && nblk >= 32 ? 16 : 4;
 }
 
-// Time chunks of the lane-per-state mapping: one where the rows give each of the 1024 SIMDs 3
+// Time chunks of the lane-per-state mapping: one where the rows give each of the 1024 SIMDs 2
 // wavefronts, else the smallest power of two that gives them 4 (as many as bwd_lane's LDS and
 // registers allow), with at least four blocks each, and past 64 chunks at least half as many blocks
 // as there are chunks, since every chunk composes the maps of those beside it.  A chunk costs its
 // map and, in the backward, its own dA / dD / ddelta_bias partials.  us a backward, bf16, splitting
 // up to 3 wavefronts a SIMD / 4 / 6: 768 rows x 4096 steps 90 / 88 / 86, 1536 x 4096 167 / 159 / 163,
-// 3072 x 2048 171 / 164 / 169, 3072 x 8192 609 / 584 / 592; 12288 x 1024, which has 3 from its rows,
-// 234 in one chunk, 257 in two.  At 131072 steps with at most 64 chunks / as here: 4 rows 267 / 123,
+// 3072 x 2048 171 / 164 / 169, 3072 x 8192 609 / 584 / 592.  8192 rows, which are 2, in one chunk and
+// in two: 72 / 75 at 256 steps, 182 / 182 at 1024.  At 131072 steps with at most 64 chunks / as here: 4 rows 267 / 123,
 // 64 rows 314 / 247, 256 rows 894 / 808.
 static int lane_time_chunks(const Geo& g) {
   const int64_t quads = g.rows / kLaneChannels;
   const int64_t nblk = (g.length + HS - 1) / HS;
   int64_t k = 1;
-  if (quads < 3072)
+  if (quads < 2048)
     while (quads * k < 4096 && nblk >= 8 * k && (k < 64 || nblk >= k * k / 2)) k <<= 1;
   const int64_t per = (nblk + k - 1) / k;
   return static_cast<int>((nblk + per - 1) / per);
@@ -2267,21 +2274,21 @@ static bool chain_by_wave(const Geo& g) {
 }
 
 
-template <class TU, class TB, bool VBC, bool RESTART>
+template <class TU, class TB, bool VBC, Walk WALK>
 static void launch_fwd_lane_t(const Geo& g, const Ptrs& q, hipStream_t s) {
-  const int k = g.nchunks > 1 ? 1 : lane_chunks(g);
-  const int64_t quads = g.rows / kLaneChannels;
-  const dim3 grid(blocks_for(quads, k == 1 ? 4 : 1), g.nchunks);
-  if constexpr (!RESTART) {
-    if (g.nchunks > 1)
-      MKO_TIMED("selscan_fwd_map", s, fwd_map<TU, TB, VBC><<<dim3(grid.x, g.nchunks - 1), 256, 0, s>>>(g, q));
+  const unsigned quads = blocks_for(g.rows, kLaneChannels);
+  const int k = lane_chunks(g);
+  if constexpr (WALK == CHUNKS) {
+    const unsigned gx = blocks_for(quads, 4);
+    MKO_TIMED("selscan_fwd_map", s, fwd_map<TU, TB, VBC><<<dim3(gx, g.nchunks - 1), 256, 0, s>>>(g, q));
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, WALK><<<dim3(gx, g.nchunks), 256, 0, s>>>(g, q));
+  } else if (k == 1) {
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, WALK><<<blocks_for(quads, 4), 256, 0, s>>>(g, q));
+  } else if (k == 4) {
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4, WALK><<<quads, 256, 0, s>>>(g, q));
+  } else {
+    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16, WALK><<<quads, 1024, 0, s>>>(g, q));
   }
-  if (k == 1)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 1, RESTART><<<grid, 256, 0, s>>>(g, q));
-  else if (k == 4)
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 4, RESTART><<<grid, 256, 0, s>>>(g, q));
-  else
-    MKO_TIMED("selscan_fwd_lane", s, fwd_lane<TU, TB, VBC, 16, RESTART><<<grid, 1024, 0, s>>>(g, q));
 }
 
 template <class TU>
@@ -2294,13 +2301,17 @@ static int launch_fwd_lane(const Plan& pl, const Ptrs& q0, const mko_selscan_par
   q.drive = static_cast<float*>(p->workspace);
   q.sumd = reinterpret_cast<float*>(static_cast<char*>(p->workspace) + pl.foff_sumd);
   // chunks are of sequences past kRestartSteps (128 blocks and more)
-  const bool restart = g.nchunks == 1 && !(pl.vbc && full_walk(g)) && g.length <= kRestartSteps;
-  auto go = [&](auto tb) {
+  const Walk walk = g.nchunks > 1 ? CHUNKS : (!(pl.vbc && full_walk(g)) && g.length <= kRestartSteps ? RESTARTS : WHOLE);
+  auto go_v = [&](auto tb, auto vbc) {
     using TB = decltype(tb);
-    if (pl.vbc && restart) launch_fwd_lane_t<TU, TB, true, true>(g, q, s);
-    else if (pl.vbc) launch_fwd_lane_t<TU, TB, true, false>(g, q, s);
-    else if (restart) launch_fwd_lane_t<TU, TB, false, true>(g, q, s);
-    else launch_fwd_lane_t<TU, TB, false, false>(g, q, s);
+    constexpr bool VBC = decltype(vbc)::value;
+    if (walk == CHUNKS) launch_fwd_lane_t<TU, TB, VBC, CHUNKS>(g, q, s);
+    else if (walk == RESTARTS) launch_fwd_lane_t<TU, TB, VBC, RESTARTS>(g, q, s);
+    else launch_fwd_lane_t<TU, TB, VBC, WHOLE>(g, q, s);
+  };
+  auto go = [&](auto tb) {
+    if (pl.vbc) go_v(tb, std::true_type{});
+    else go_v(tb, std::false_type{});
   };
   if (g.bc_dtype == MKO_BF16) go(bf16{});
   else if (g.bc_dtype == MKO_F16) go(_Float16{});
