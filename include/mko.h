@@ -138,9 +138,10 @@ size_t mko_selscan_bwd_workspace_size(const mko_selscan_params* p);
 int mko_selscan_bwd(const mko_selscan_params* p, void* stream);
 
 /* Which mapping each direction takes for this geometry: 1 for the lane-per-(channel, state)
- * kernels, 0 for the lane-per-channel ones.
- * Host only, no launch; pointers are not read.  No reference counterpart (the reference
- * has one Metal mapping). */
+ * kernels, 0 for the lane-per-channel ones.  For 16-byte aligned rows: some calls of narrow
+ * states that leave the lane-per-(channel, state) kernels stay on them when a row is not
+ * aligned.  Host only, no launch; of the pointers only whether z is set is looked at.  No
+ * reference counterpart (the reference has one Metal mapping). */
 int mko_selscan_plan(const mko_selscan_params* p, int* fwd_lane, int* bwd_lane);
 
 /* ======================================================================== */

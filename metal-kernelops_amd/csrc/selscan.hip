@@ -2027,7 +2027,7 @@ struct Plan {
   Geo g;
   int ns;
   bool uni;
-  bool lane;  // forward through fwd_lane (set per call from pointer alignment and shape)
+  bool lane;  // forward through fwd_lane (set per call from shape and pointer alignment)
   bool vbc;   // fwd_lane reads B and C as vectors
   bool lane_bwd;  // backward through bwd_lane (likewise)
   size_t off_bt, off_ct, off_bn, off_cn, off_drive, off_sumd, off_adj, off_pbc, off_dap, off_ddp,
@@ -2064,6 +2064,31 @@ static int lane_chunks(const Geo& g) {
   const int64_t nblk = (g.length + HS - 1) / HS;
   if (quads >= 1536 || nblk < 4) return 1;
   return quads <= 384 && nblk >= 32 ? 16 : 4;
+}
+
+// Narrow states leave lanes of the lane-per-state kernels idle, whose time does not depend on dstate,
+// while the lane-per-channel kernels walk the states there are: where these fill the chip and their
+// loads are typed (whole blocks of aligned rows, groups of a multiple of 64 channels), enough work
+// outweighs their further launches.  Both directions compare the two in us per 10^6 element-steps, a
+// launch cost against the difference of the rates.  Backward, bf16 with a gate, lane per state /
+// per channel: 3072 rows x 4096 steps, dstate 1 281 / 196, 4 283 / 231, 8 294 / 284; 1536 x 2048,
+// dstate 1 86 / 77, 4 90 / 96; 16 states 302 / 365 at 3072 x 4096.  Without a gate the lane-per-state
+// backward has less to do (fp32, 1536 x 3136, dstate 1 108 / 96; x 12544, dstate 8 362 / 472).  Forward: 1536 x 8192, whose 16 runs
+// take the CUs two rounds, dstate 1 146 / 125, 4 149 / 137, 8 149 / 155; 3072 x 8192, dstate 1 222 / 211,
+// 4 224 / 226.  From 4096 rows (forward) and kLaneRows (backward) on the lane-per-state kernels stay.
+static bool per_channel_fwd(const Geo& g) {
+  if (g.rows >= 4096) return false;
+  const double work = 1e-6 * static_cast<double>(g.rows) * static_cast<double>(g.length);
+  const double per_state = g.rows > 1024 && g.rows <= 1536 ? 11.4 : 9.0;
+  return (per_state - 7.2 - 0.3 * static_cast<double>(g.dstate)) * work > 35.0;
+}
+static bool per_channel_bwd(const Geo& g, bool gate) {
+  if (g.rows >= kLaneRows) return false;
+  const double work = 1e-6 * static_cast<double>(g.rows) * static_cast<double>(g.length);
+  const double n = static_cast<double>(g.dstate);
+  // fewer than 256 rows fill the chip later
+  const double launches = (gate ? 22.0 : 11.0) * std::max(1.0, 256.0 / static_cast<double>(g.rows));
+  return (gate ? 9.0 - 0.8 * n : 3.5 - 0.9 * n) * work > launches;
 }
 
 // Time chunks of the lane-per-state mapping: one where the rows give each of the 1024 SIMDs 2
@@ -2451,8 +2476,10 @@ extern "C" int mko_selscan_plan(const mko_selscan_params* p, int* fwd_lane, int*
   Plan pl;
   const int st = make_plan(p, &pl);
   if (st != MKO_OK) return st;
-  if (fwd_lane) *fwd_lane = lane_shape(pl.g, pl.ns) ? 1 : 0;
-  if (bwd_lane) *bwd_lane = lane_bwd_shape(pl.g, pl.ns) ? 1 : 0;
+  const Geo& g = pl.g;
+  const bool typed = pl.uni && g.length % HS == 0 && (g.length * dtype_size(p->u_dtype)) % 16 == 0;
+  if (fwd_lane) *fwd_lane = lane_shape(g, pl.ns) && !(typed && per_channel_fwd(g)) ? 1 : 0;
+  if (bwd_lane) *bwd_lane = lane_bwd_shape(g, pl.ns) && !(typed && per_channel_bwd(g, p->z != nullptr)) ? 1 : 0;
   return MKO_OK;
 }
 
@@ -2471,7 +2498,7 @@ extern "C" int mko_selscan_fwd(const mko_selscan_params* p, void* stream) {
   }
   pl.g.vec = rows_vectorisable(pl.g, {{p->u, p->u_dtype}, {p->delta, p->delta_dtype}, {p->z, p->u_dtype},
                                       {p->out, p->u_dtype}}) ? 1 : 0;
-  pl.lane = lane_shape(pl.g, pl.ns);
+  pl.lane = lane_shape(pl.g, pl.ns) && !(pl.uni && pl.g.vec && pl.g.length % HS == 0 && per_channel_fwd(pl.g));
   pl.vbc = rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
   Ptrs q = make_ptrs(p, pl);
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2507,7 +2534,8 @@ extern "C" int mko_selscan_bwd(const mko_selscan_params* p, void* stream) {
   pl.g.vec = rows_vectorisable(pl.g, {{p->u, p->u_dtype}, {p->delta, p->delta_dtype}, {p->z, p->u_dtype},
                                       {p->dout, p->u_dtype}, {p->du, p->u_dtype}, {p->ddelta, p->delta_dtype},
                                       {p->dz, p->u_dtype}, {p->out, p->u_dtype}}) ? 1 : 0;
-  pl.lane_bwd = lane_bwd_shape(pl.g, pl.ns);
+  pl.lane_bwd = lane_bwd_shape(pl.g, pl.ns) &&
+                !(pl.uni && pl.g.vec && pl.g.length % HS == 0 && per_channel_bwd(pl.g, p->z != nullptr));
   pl.vbc = rows_vectorisable(pl.g, {{p->B, p->bc_dtype}, {p->C, p->bc_dtype}});
   Ptrs q = make_ptrs(p, pl);
   hipStream_t s = static_cast<hipStream_t>(stream);

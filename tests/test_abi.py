@@ -156,3 +156,27 @@ def test_lane_backward_refused_past_its_32_bit_offsets(native):
     assert plan(1, 8192, 65536, 512) == (1, 1)
     # rows * length itself at 2^31
     assert plan(1, 8192, 262144, 1) == (1, 0)
+
+
+def test_narrow_states_leave_the_lane_per_state_kernels(native):
+    """Where narrow states leave its lanes idle and there is work enough, the lane-per-channel mapping
+    runs: both sides of the lines, and what keeps a call where it is (16 states, ragged rows, groups
+    that a wavefront does not fit, many rows)."""
+    lib = native.lib()
+
+    def plan(rows, length, dstate, groups=1, gate=True, dtype=native.BF16):
+        p = native.SelscanParams()
+        p.batch, p.dim, p.length, p.dstate, p.ngroups, p.u_dtype = 1, rows, length, dstate, groups, dtype
+        p.z = 1 if gate else None
+        fwd, bwd = ctypes.c_int(-1), ctypes.c_int(-1)
+        assert lib.mko_selscan_plan(ctypes.byref(p), ctypes.byref(fwd), ctypes.byref(bwd)) == 0
+        return fwd.value, bwd.value
+
+    assert plan(1536, 8192, 1) == (0, 0) and plan(1536, 4096, 1) == (1, 0) and plan(1536, 1024, 1) == (1, 1)
+    assert plan(1536, 8192, 4) == (0, 0) and plan(1536, 2048, 4) == (1, 1)
+    assert plan(3072, 8192, 1) == (0, 0) and plan(3072, 8192, 4) == (1, 0) and plan(5120, 1024, 8) == (1, 1)
+    assert plan(3072, 4096, 8) == (1, 0) and plan(3072, 4096, 8, gate=False) == (1, 1)
+    assert plan(64, 131072, 4) == (1, 1) and plan(128, 131072, 4) == (1, 0)
+    for stays in ((3072, 8192, 16), (1536, 65536, 16), (3072, 8200, 1), (3072, 8191, 1), (6144, 8192, 1)):
+        assert plan(*stays) == (1, 1), stays
+    assert plan(3072, 8192, 1, groups=64) == (1, 1)

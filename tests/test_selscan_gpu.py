@@ -493,3 +493,21 @@ def test_long_few_rows_keep_the_chip_busy():
     _, states = selscan_fwd_impl(*args, True)
     assert timed(lambda: selscan_fwd_impl(*args, True)) < 300
     assert timed(lambda: selscan_bwd_impl(dy, *args, True, states)) < 230
+
+
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16], ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("dstate", [1, 3, 4])
+def test_narrow_states_agree_on_both_mappings(dstate, act):
+    # Enough work of narrow states runs on the lane-per-channel mapping; the same values one element
+    # past a 16-byte boundary stay on the lane-per-state one.  float32 results agree to 2e-6 (both sit
+    # within 6e-7 of the exact ones), 16-bit ones to a rounding of theirs.
+    inputs, dy = _random_problem(1, 1536, 8192, dstate, 1, seed=dstate, act=act)
+    dev = {k: v.to(DEV) for k, v in inputs.items()}
+    moved = dev | {"u": _off_alignment(dev["u"])}
+    assert "selscan_fwd_replay" in _forward_kernels(dev, True) and "selscan_fwd_lane" in _forward_kernels(moved, True)
+    dy = dy.to(DEV)
+    assert "selscan_bwd_main" in _backward_kernels(dev, dy) and "selscan_bwd_lane" in _backward_kernels(moved, dy)
+    (a, da), (b, db) = _gpu(dev, dy), _gpu(moved, dy)
+    for name, x, y in [("out", a, b)] + [(k, da[k], db[k]) for k in NAMES]:
+        tol = 2e-6 if x.dtype == torch.float32 else 4e-3
+        assert norm_rel(x, y) <= tol, (name, norm_rel(x, y))
