@@ -367,18 +367,33 @@ chunk_state(Geo g, Ptrs p, void* out_, int ncb) {
   }
 }
 
+// Workgroups of 256 threads one launch may have: a grid of 2^32 threads and more is cut off modulo
+// 2^32 without an error.  Two kinds of workgroups share a launch only within it.
+constexpr int64_t kMaxWgs = (int64_t{1} << 32) / 256 - 1;
+
 template <typename TM, bool VEC, bool BWD>
 inline void launch_chunk_state(const Geo& g, const Ptrs& q, void* out, hipStream_t s) {
-  const int ncb = BWD ? 0 : static_cast<int>(g.qb * (g.qb + 1) / 2 * g.nc * g.ngroups * g.batch);
-  const dim3 grid(static_cast<unsigned>(ncb + g.npt * g.nnp * g.nc * g.batch * g.nheads));
+  const int64_t ncb = BWD ? 0 : static_cast<int64_t>(g.qb * (g.qb + 1) / 2) * g.nc * g.ngroups * g.batch;
+  const int64_t ncs = static_cast<int64_t>(g.npt * g.nnp) * g.nc * g.batch * g.nheads;
   const char* name = BWD ? "ssd_chunk_state_bwd" : "ssd_chunk_state";
-  if constexpr (sizeof(TM) == 2) {
-    if (g.qb == 4) {
-      MKO_TIMED(name, s, chunk_state<TM, VEC, BWD, 4><<<grid, 256, 0, s>>>(g, q, out, ncb));
-      return;
+  // the first `tiles` of `wgs` workgroups are C.B^T tiles
+  auto go = [&](int64_t tiles, int64_t wgs) {
+    const dim3 grid(static_cast<unsigned>(wgs));
+    const int n = static_cast<int>(tiles);
+    if constexpr (sizeof(TM) == 2) {
+      if (g.qb == 4) {
+        MKO_TIMED(name, s, chunk_state<TM, VEC, BWD, 4><<<grid, 256, 0, s>>>(g, q, out, n));
+        return;
+      }
     }
+    MKO_TIMED(name, s, chunk_state<TM, VEC, BWD><<<grid, 256, 0, s>>>(g, q, out, n));
+  };
+  if (ncb + ncs <= kMaxWgs) {
+    go(ncb, ncb + ncs);
+  } else {
+    if (ncb > 0) go(ncb, ncb);
+    go(0, ncs);
   }
-  MKO_TIMED(name, s, chunk_state<TM, VEC, BWD><<<grid, 256, 0, s>>>(g, q, out, ncb));
 }
 
 // Loads cs and step of a whole chunk into LDS (q <= 256 values each), and the column

@@ -1280,14 +1280,13 @@ dbc_state(Geo g, BwdPlan pl, Ptrs p, int nst_wgs) {
 }
 
 // dC = dCB B (which 1) and dB = dCB^T C (which 0) for one 64-token tile and two
-// d_state tiles, plus the head-block partials of the state terms.  The launch's first nheads
+// d_state tiles, plus the head-block partials of the state terms.  The launch's first `heads`
 // workgroups are reduce_head's.
 template <typename TM, bool VEC>
-__global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p) {
+__global__ void __launch_bounds__(256) dbc_final(Geo g, BwdPlan pl, Ptrs p, int heads) {
   constexpr int TE = LdsTile<TM>::elems;
   constexpr int NB = kStageBufs<TM>;
   __shared__ __align__(16) TM sbuf[NB][3 * TE];
-  const int heads = static_cast<int>(g.nheads);
   if (static_cast<int>(blockIdx.x) < heads) {
     reduce_head(g, p, blockIdx.x);
     return;
@@ -1573,9 +1572,17 @@ int launch_bwd_t(const Geo& g, const BwdPlan& pl, const Ptrs& q, hipStream_t s) 
   MKO_TIMED("ssd_state_rev", s, state_rev<TM><<<dim3(pl.nblk, bh), 256, 0, s>>>(g, pl, q));
   launch_du<TM, VEC>(g, pl, q, s);
   if (!join) dcb(s);
-  const unsigned nst_wgs = g.qb * g.nnp * 2 * pl.hb2 * ncg * nb;
-  MKO_TIMED("ssd_dbc_state", s,
-            dbc_state<TM, VEC><<<dim3(nst_wgs + g.nc * bh), 256, 0, s>>>(g, pl, q, static_cast<int>(nst_wgs)));
+  const int64_t nst_wgs = static_cast<int64_t>(g.qb * g.nnp * 2 * pl.hb2) * ncg * nb, nfin = static_cast<int64_t>(g.nc) * bh;
+  auto dbc = [&](int64_t states, int64_t wgs) {  // the first `states` workgroups, then finish's
+    MKO_TIMED("ssd_dbc_state", s,
+              dbc_state<TM, VEC><<<dim3(static_cast<unsigned>(wgs)), 256, 0, s>>>(g, pl, q, static_cast<int>(states)));
+  };
+  if (nst_wgs + nfin <= kMaxWgs) {
+    dbc(nst_wgs, nst_wgs + nfin);
+  } else {
+    dbc(nst_wgs, nst_wgs);
+    dbc(0, nfin);
+  }
   if (join) {
     const hipError_t e = hipStreamWaitEvent(s, join, 0);
     if (e != hipSuccess) {
@@ -1583,8 +1590,14 @@ int launch_bwd_t(const Geo& g, const BwdPlan& pl, const Ptrs& q, hipStream_t s) 
       return MKO_ELAUNCH;
     }
   }
+  const int64_t nfinal = static_cast<int64_t>(g.qb * g.nnp * 2) * ncg * nb;
+  int heads = static_cast<int>(g.nheads);
+  if (nfinal + heads > kMaxWgs) {
+    MKO_TIMED("ssd_reduce", s, reduce_params<<<dim3(static_cast<unsigned>(heads)), 256, 0, s>>>(g, q));
+    heads = 0;
+  }
   MKO_TIMED("ssd_dbc_final", s,
-            dbc_final<TM, VEC><<<dim3(static_cast<unsigned>(g.nheads) + g.qb * g.nnp * 2 * ncg * nb), 256, 0, s>>>(g, pl, q));
+            dbc_final<TM, VEC><<<dim3(static_cast<unsigned>(nfinal + heads)), 256, 0, s>>>(g, pl, q, heads));
   return MKO_OK;
 }
 

@@ -572,3 +572,32 @@ def test_double_backward_is_refused():
     (gx,) = torch.autograd.grad((y * dy.to(DEV).float()).sum(), leaves["x"], create_graph=True)
     with pytest.raises(RuntimeError):
         gx.sum().backward()
+
+
+def test_grids_that_fit_alone_but_not_together():
+    # 4095 x 4096 single-token sequences: 16,773,120 chunk states and as many of the backward's last
+    # sums, within a launch's 2^24 - 1 workgroups of 256 threads, but not together with the C.B^T
+    # tiles (16380) or the state terms of dB and dC.  One token has closed forms: the state is
+    # dt x (x) B and y = dt x (B.C); B and C are positive, so that every sum is far from zero.
+    from metal_kernelops.cv import mamba2_chunk_scan
+    batch, heads, groups = 4095, 4096, 4
+    rep = heads // groups
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(batch, 1, heads, 1, device=DEV, generator=g)
+    dt = torch.rand(batch, 1, heads, device=DEV, generator=g) + 0.1
+    A = -torch.rand(heads, device=DEV, generator=g)
+    B, C = (torch.rand(batch, 1, groups, 1, device=DEV, generator=g) + 0.5 for _ in range(2))
+    leaves = [t.requires_grad_(True) for t in (x, dt, A, B, C)]
+    y, final = mamba2_chunk_scan(*leaves)
+    grads = torch.autograd.grad(y, leaves, torch.ones_like(y))
+    with torch.no_grad():
+        bh, ch = (t[:, 0, :, 0].repeat_interleave(rep, 1) for t in (B, C))
+        xs, steps = x[:, 0, :, 0], dt[:, 0]
+        term = (steps * xs).view(batch, groups, rep).sum(-1)
+        want = {"y": (y[:, 0, :, 0], steps * xs * bh * ch), "final": (final[:, :, 0, 0], steps * xs * bh),
+                "dx": (grads[0][:, 0, :, 0], steps * bh * ch), "ddt": (grads[1][:, 0], xs * bh * ch),
+                "dB": (grads[3][:, 0, :, 0], term * C[:, 0, :, 0]), "dC": (grads[4][:, 0, :, 0], term * B[:, 0, :, 0])}
+        for name, (got, ref) in want.items():
+            err = ((got - ref).norm() / ref.norm()).item()
+            assert err <= 1e-5, (name, err)
+        assert grads[2].abs().max().item() <= 1e-3  # no decay reaches a single token's output
