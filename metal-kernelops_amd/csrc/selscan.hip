@@ -1,8 +1,8 @@
 // Mamba-1 selective scan, forward and backward, for gfx950.
 //
-// Two mappings.  dstate <= 16 with groups of a multiple of 4 channels runs one lane per
-// (channel, state): fwd_lane and bwd_lane, below.  What follows is the other one, for wider
-// states and odd groups.
+// Two mappings.  dstate <= 16 with groups of a multiple of 4 channels and fp32 step sizes runs one
+// lane per (channel, state): fwd_lane and bwd_lane, below.  What follows is the other one, for wider
+// states, odd groups, 16-bit step sizes and much work of few states (per_channel_fwd).
 //
 // Mapping: one lane per channel row (batch, d).  A wavefront holds 64 channels of
 // one (batch, group) whenever dim/ngroups is a multiple of 64 ("uniform" mode), so
@@ -2123,10 +2123,10 @@ static int lane_fwd_chunks(const Geo& g) {
 // 1325 us against 1503 with the sum, 8 x 1536 x 2048 386 against 460).
 static bool full_walk(const Geo& g) { return g.rows >= kLaneRows && g.vec && g.length % HS == 0; }
 
-// The backward's too.  It indexes the per-row arrays (u, delta, z, dout, out, du, ddelta, dz,
-// the saved states) and B/C with 32-bit lane offsets from a 64-bit base, so each of them must
-// hold fewer than 2^31 elements: rows x length for the rows, and batch x groups x 16 states x
-// length for B and C (four times the rows' count when a group is 4 channels wide).
+// The backward's too, below 2^31 elements in the rows and in B and C (which hold four times as many
+// as the rows when a group is 4 channels wide).  Its offsets are 64-bit from row to row and would
+// reach further; past that size (8.6 GB of step sizes) it has not been run, and the lane-per-channel
+// kernels take the call.
 static bool lane_bwd_shape(const Geo& g, int ns) {
   constexpr int64_t kLimit = static_cast<int64_t>(1) << 31;
   return lane_shape(g, ns) && g.rows * g.length < kLimit && g.batch * g.ngroups * HS * g.length < kLimit;

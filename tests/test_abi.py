@@ -133,10 +133,11 @@ def test_static_decode_backward_refuses_an_oversized_problem_on_the_host(native)
 
 
 def test_lane_backward_refused_past_its_32_bit_offsets(native):
-    """The lane-per-state backward addresses B/C with 32-bit lane offsets.  With groups of
-    4 channels B/C hold four times as many elements as u, so a geometry whose rows x length
-    still fits 2^31 while batch x groups x 16 x length does not must plan the
-    lane-per-channel backward; the forward (64-bit offsets) keeps its lane mapping."""
+    """The lane-per-state backward is kept to fewer than 2^31 elements in the rows and in B/C, the
+    range it has been run over (its offsets would reach further).  With groups of 4 channels B/C
+    hold four times as many elements as u, so a geometry whose rows x length still fits 2^31
+    while batch x groups x 16 x length does not must plan the lane-per-channel backward; the
+    forward keeps its lane mapping."""
     lib = native.lib()
 
     def plan(batch, dim, length, groups):

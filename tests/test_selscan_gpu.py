@@ -93,12 +93,14 @@ def _random_problem(batch, dim, length, dstate, groups, seed, act=torch.float32,
 
 
 SHAPES = [
-    (2, 8, 64, 16, 2),      # config 1 geometry, lanes span groups (atomic dB/dC path)
-    (2, 128, 200, 16, 2),   # one 64-channel wavefront per group, ragged length
-    (1, 256, 300, 16, 1),   # four wavefronts per workgroup, several coarse chunks
+    # lane per (channel, state)
+    (2, 8, 64, 16, 2),      # config 1 geometry: groups of one wavefront's 4 channels
+    (2, 128, 200, 16, 2),   # 16-channel dB/dC partials, ragged length
+    (1, 256, 300, 16, 1),   # time split over 4 wavefronts (forward) and in chunks (backward)
     (2, 64, 97, 5, 1),      # dstate padded to 16
-    (1, 128, 130, 32, 2),   # dstate 32
-    (3, 24, 77, 20, 3),     # dstate 20, ragged everything
+    # lane per channel
+    (1, 128, 130, 32, 2),   # dstate 32, one 64-channel wavefront per group
+    (3, 24, 77, 20, 3),     # dstate 20, ragged everything, wavefronts across groups
 ]
 
 
@@ -134,10 +136,10 @@ def test_bf16_delta_and_fp16():
     _compare(inputs, dy, True, "1x128x200 bf16 with bf16 delta")
 
 
-# At 6144 channels (batch x dim) and more, dstate <= 16 and whole 16-step blocks, the forward
-# runs one lane per (channel, state) over the whole sequence; its saved states feed the backward.
+# At 6144 channels (batch x dim) and more and whole blocks of aligned rows, each wavefront of the
+# lane-per-state kernels walks the whole sequence; its saved states feed the backward.
 LANE_SHAPES = [
-    (2, 3072, 64, 16, 1),   # the smallest lane-path problem
+    (2, 3072, 64, 16, 1),   # the smallest such problem
     (2, 3072, 48, 12, 2),   # dstate 12 (lanes 12..15 idle), two groups
     (1, 6200, 32, 16, 2),   # a ragged last workgroup, two groups of 3100 channels
     (2, 3072, 16, 16, 1),   # one 16-step block: the backward's load ahead re-reads block 0
@@ -186,7 +188,7 @@ def _backward_kernels(inputs, dy, softplus=True):
                                    (2, 3072, 16, 16, 1)],
                          ids=["groups-of-3072", "groups-of-3100", "dstate-12-groups-of-1024", "one-16-step-block"])
 def test_lane_backward_kernel_is_taken_and_deterministic(shape):
-    # 6144+ channel rows, whole 16-step blocks, dstate <= 16 and groups a multiple of 4
+    # 6144+ channel rows in whole 16-step blocks, dstate <= 16 and groups a multiple of 4
     # channels wide: one lane per (channel, state) walks the sequence backwards. Groups of a
     # multiple of 16 channels add their dB/dC in 16-channel workgroup partials, others in
     # 4-channel wavefront partials; both orders are fixed.
@@ -262,16 +264,18 @@ def test_lane_forward_16bit():
 @pytest.mark.parametrize("shape", [(1, 64, 2000, 16, 1), (2, 24, 1500, 20, 3)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_long_sequences_few_channels(shape):
-    # Few rows and 16-step chunks: 125 (94) chunks, more than 32, so the chunk chains run
-    # a wavefront per (row, state) with the chunks split into runs across its lanes.
+    # 64 rows of 16 states: 16 runs of a workgroup's wavefronts (forward), 16 chunks (backward).
+    # 20 states take the lane-per-channel kernels, in 16-step chunks: 94 of them, more than 32, so
+    # the chunk chains run a wavefront per (row, state) with the chunks split into runs across its
+    # lanes (with 16 states: test_sixteen_states_on_the_lane_per_channel_kernels).
     inputs, dy = _random_problem(*shape, seed=sum(shape))
     _compare(inputs, dy, True, "long " + "x".join(map(str, shape)))
 
 
 def test_partial_reductions_whole_batches_and_tail():
-    # One group of 2304 channels: 9 blocks of 256 channels feed each dB/dC value (a batch
-    # of eight partials plus one), and the 256 steps run as 16 chunks of 16, so each
-    # dA/dD/ddelta_bias value sums 16 chunks x 2 batches = 32 partials in whole batches.
+    # One group of 2304 channels: 144 partials of 16 channels feed each dB/dC value, nine whole
+    # batches of sixteen.  The lane-per-channel kernels' own partials (9 blocks of 256 channels, 32
+    # of dA in whole batches) are in test_sixteen_states_on_the_lane_per_channel_kernels.
     inputs, dy = _random_problem(2, 2304, 256, 16, 1, seed=23)
     _compare(inputs, dy, True, "2x2304x256")
 
@@ -380,26 +384,49 @@ def test_lane_time_splits_and_ragged_rows(shape, act):
     _compare(inputs, dy, True, "split " + "x".join(map(str, shape)) + f" {act}")
 
 
-@pytest.mark.parametrize("length", [37, 531])
-def test_ragged_rows_keep_apart(length):
-    # A ragged row's last block reads on into the next row: nothing of it may come back.  Channel 5
-    # is NaN throughout, and so are B's and C's last states; every other channel must match a run
-    # without them.
-    inputs, dy = _random_problem(1, 8, length, 16, 2, seed=3)
-    clean = _gpu(inputs, dy, True)
-    bad = {k: v.clone() for k, v in inputs.items()}
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16], ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("length", [37, 531, 2055])
+def test_ragged_rows_keep_apart(length, act):
+    # A ragged row's last block reads on into the next row, of the same wavefront (channel 0 into 1,
+    # state 0 into 1) or of the next group (state 4 of group 0 into group 1): nothing of it may come
+    # back.  Each such neighbour is NaN in turn, and what does not depend on it must keep its bits.
+    # 5 states and odd lengths leave 16-bit rows of group 1 on 2-byte boundaries.
+    inputs, dy = _random_problem(1, 8, length, 5, 2, seed=3, act=act)
+    out, grads = _gpu(inputs, dy, True)
+
+    def poisoned(where):
+        bad = {k: v.clone() for k, v in inputs.items()}
+        for k, index in where.items():
+            bad[k][index] = float("nan")
+        return _gpu(bad, dy, True)
+
+    # channel 1's rows: every other channel, and group 1's dB and dC
+    others = [0, 2, 3, 4, 5, 6, 7]
+    got, g = poisoned({k: (0, 1) for k in ("u", "dt", "z")})
+    assert torch.equal(got[:, others], out[:, others])
     for k in ("u", "dt", "z"):
-        bad[k][0, 5] = float("nan")
-    for k in ("B", "C"):
-        bad[k][0, 1] = float("nan")
-    out, grads = _gpu(bad, dy, True)
-    assert torch.equal(out[:, :4], clean[0][:, :4])
-    for k in ("u", "dt", "z"):
-        assert torch.equal(grads[k][:, :4], clean[1][k][:, :4]), k
-    for k in ("B", "C"):
-        assert torch.equal(grads[k][:, 0], clean[1][k][:, 0]), k
+        assert torch.equal(g[k][:, others], grads[k][:, others]), k
     for k in ("A", "D", "delta_bias"):
-        assert torch.equal(grads[k][:4], clean[1][k][:4]), k
+        assert torch.equal(g[k][others], grads[k][others]), k
+    for k in ("B", "C"):
+        assert torch.equal(g[k][:, 1], grads[k][:, 1]), k
+    # state 1 of group 0: the other states' dA, dB and dC, and all of group 1
+    got, g = poisoned({"B": (0, 0, 1), "C": (0, 0, 1)})
+    states = [0, 2, 3, 4]
+    assert torch.equal(g["A"][:4, states], grads["A"][:4, states])
+    assert torch.equal(got[:, 4:], out[:, 4:]) and torch.equal(g["A"][4:], grads["A"][4:])
+    for k in ("B", "C"):
+        assert torch.equal(g[k][:, 0, states], grads[k][:, 0, states]), k
+        assert torch.equal(g[k][:, 1], grads[k][:, 1]), k
+    # group 1's first state: all of group 0
+    got, g = poisoned({"B": (0, 1, 0), "C": (0, 1, 0)})
+    assert torch.equal(got[:, :4], out[:, :4])
+    for k in ("u", "dt", "z"):
+        assert torch.equal(g[k][:, :4], grads[k][:, :4]), k
+    for k in ("A", "D", "delta_bias"):
+        assert torch.equal(g[k][:4], grads[k][:4]), k
+    for k in ("B", "C"):
+        assert torch.equal(g[k][:, 0], grads[k][:, 0]), k
 
 
 def _off_alignment(t):
@@ -511,3 +538,39 @@ def test_narrow_states_agree_on_both_mappings(dstate, act):
     for name, x, y in [("out", a, b)] + [(k, da[k], db[k]) for k in NAMES]:
         tol = 2e-6 if x.dtype == torch.float32 else 4e-3
         assert norm_rel(x, y) <= tol, (name, norm_rel(x, y))
+
+
+# Step sizes of 16 bits, which the library takes and the wrapper widens, stay on the lane-per-channel
+# kernels with 16 states: uniform wavefronts with a ragged length; four wavefronts a workgroup and
+# several coarse chunks; 125 chunks, chained by a wavefront per (row, state); 9 blocks of 256
+# channels to a dB/dC value and 32 partials to one of dA; wavefronts across groups.
+CHANNEL_SHAPES = [(2, 128, 200, 16, 2), (1, 256, 300, 16, 1), (1, 64, 2000, 16, 1), (2, 2304, 256, 16, 1),
+                  (2, 24, 77, 16, 3)]
+
+
+@pytest.mark.parametrize("delta", [torch.bfloat16, torch.float16], ids=lambda t: str(t).split(".")[-1])
+@pytest.mark.parametrize("shape", CHANNEL_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_sixteen_states_on_the_lane_per_channel_kernels(shape, delta):
+    if shape[1] > 2000 and delta != torch.bfloat16:
+        pytest.skip("one type at the widest: its oracle takes seconds")
+    from metal_kernelops import _native as nat
+    from metal_kernelops.scan import selscan_bwd_impl, selscan_fwd_impl
+    inputs, dy = _random_problem(*shape, seed=sum(shape) + 11)
+    inputs["dt"] = inputs["dt"].to(delta)
+    args = [inputs[k].to(DEV) for k in NAMES]
+    nat.kernel_timing_reset()
+    nat.kernel_timing(True)
+    try:
+        out, states = selscan_fwd_impl(*args, True)
+        grads = selscan_bwd_impl(dy.to(DEV), *args, True, states)
+        torch.cuda.synchronize()
+        kernels = set(nat.kernel_times())
+    finally:
+        nat.kernel_timing(False)
+    assert {"selscan_fwd_replay", "selscan_bwd_main"} <= kernels and not any("lane" in k for k in kernels), kernels
+    ref, want = _ref(inputs, dy, True)
+    assert max_rel(out, ref) <= 1e-5
+    for name, got in zip(NAMES, grads):
+        tol = GRAD_TOL[got.dtype]
+        e = record("channel " + "x".join(map(str, shape)), "d" + name, norm_rel(got, want[name]), tol)
+        assert e <= tol, f"d{name}: {e:.3e}"
