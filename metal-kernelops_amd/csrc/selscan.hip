@@ -1286,6 +1286,7 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
       if (c0 - q > ch) carry = fmaf(fast_exp2(a2 * e[q]), carry, m[q]);
   }
   float dA_acc = 0.0f, dA_run = 0.0f, dD_acc = 0.0f, db_acc = 0.0f;
+  float dD_run = 0.0f, db_run = 0.0f;  // all three summed over 8 blocks at a time
   const float act = active ? 1.0f : 0.0f;
 
   for (int k = ke - 1; k >= kb; --k) {
@@ -1413,8 +1414,15 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
     const float duo = fmaf(del, s1, Dd * gy);
     float dd = fmaf(uu, s1, s2);
     if (g.softplus) dd *= softplus_grad_from_value(del);
-    dD_acc = fmaf(gy, uu, dD_acc);
-    db_acc = fmaf(dd, act, db_acc);
+    // 8192 x 780 fp32 in one chunk, without the runs: dD 1.12 and ddelta_bias 1.02 times their
+    // errors on the lane-per-channel mapping's short chunks; 0.81 and 0.98 with them
+    dD_run = fmaf(gy, uu, dD_run);
+    db_run = fmaf(dd, act, db_run);
+    if (k % 8 == 0) {
+      dD_acc += dD_run;
+      db_acc += db_run;
+      dD_run = db_run = 0.0f;
+    }
     if (active && ok) {
       duw[eoff + t0] = from_f32<TU>(duo);
       ddw[eoff + t0] = dd;
@@ -1452,8 +1460,8 @@ bwd_lane(Geo g, Ptrs p, int cpb) {
     }
   }
   if (active && sn) p.dap[(static_cast<int64_t>(ch) * HS + n) * g.rows + row0 + cl] = dA_acc + dA_run;
-  dD_acc = row16_sum(dD_acc);
-  db_acc = row16_sum(db_acc);
+  dD_acc = row16_sum(dD_acc + dD_run);
+  db_acc = row16_sum(db_acc + db_run);
   if (active && n == 0) {
     p.ddp[ch * g.rows + row0 + cl] = dD_acc;
     p.dbp[ch * g.rows + row0 + cl] = db_acc;
