@@ -334,7 +334,8 @@ def ssd_flops(batch, length, nheads, headdim, ngroups, dstate, q):
     Per token and head: P(Q+1) for the masked scores . X product, 2NP for the chunk
     state and 2NP for C . state; per token and group N(Q+1) for C . B^T.  The backward
     does two gradient contractions per forward one.  ssd_gate is element-wise here: the
-    forward saves the chunk output for it when a gradient will be taken.
+    forward saves the chunk output for it when a gradient will be taken.  The launch of
+    ssd_chunk_state holds the C . B^T tiles as well.
     """
     tok = batch * length
     P, N, H, G = headdim, dstate, nheads, ngroups
@@ -342,7 +343,7 @@ def ssd_flops(batch, length, nheads, headdim, ngroups, dstate, q):
     state = tok * H * 2 * N * P
     cb = tok * G * N * (q + 1)
     return {
-        "ssd_cb": cb, "ssd_chunk_state": state, "ssd_chunk_scan": tri_x + state,
+        "ssd_chunk_state": state + cb, "ssd_chunk_scan": tri_x + state,
         "ssd_chunk_state_bwd": state, "ssd_du": tri_x + state, "ssd_dcb": tri_x,
         "ssd_dbc_state": 2 * state, "ssd_dbc_final": 2 * cb,
     }

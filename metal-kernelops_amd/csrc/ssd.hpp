@@ -264,7 +264,8 @@ __device__ __forceinline__ void cb_tile(const Geo& g, const Ptrs& p, int64_t w, 
 // up to three stages in flight); QB = 0: qb at run time, two stages in flight (fp32: one, on a
 // single buffer, see kStageBufs; 4 x 1024 tokens, 32 heads, d_state 128: 57 -> 43 us)
 // The forward's launch also has, as its first ncb workgroups, the C.B^T tiles (cb_tile): they
-// wait for nothing and only chunk_scan reads them.  And it forms the chunk's step sizes and
+// wait for nothing, and no kernel of this launch reads them (chunk_scan and the backward's gate
+// and du do).  And it forms the chunk's step sizes and
 // decay exponents itself, one token a thread.  As three launches: 11 + 9 + 58 us at 4 x 4096
 // tokens, 64 heads, 65 together; a 1 x 1999-token prompt of 24 heads 38 -> 32 us.
 template <typename TM, bool VEC, bool BWD, int QB = 0>
