@@ -1045,7 +1045,7 @@ fwd_lane(Geo g, Ptrs p) {
 // The backward in fwd_lane's mapping: a wavefront holds 4 channels x 16 states, lane (c, n), and
 // walks a time chunk in reverse, 16 steps a block, carrying the adjoint from each block into the
 // one on its left.  With enough rows there is one chunk, the whole sequence.  Fewer rows are cut
-// into chunks (lane_bwd_chunks): bwd_map first walks every chunk but the first with the adjoint
+// into chunks (lane_time_chunks): bwd_map first walks every chunk but the first with the adjoint
 // alone, from a zero exit, which with the chunk's sum of steps gives its map from the adjoint
 // entering it on the right to the one leaving it on the left; bwd_lane composes the maps of
 // the chunks to the right of its own before its first block.  Unless FULL, the adjoint is carried
