@@ -493,35 +493,6 @@ def test_long_sequences_in_time_chunks(shape, act):
     _compare(inputs, dy, True, "chunks " + "x".join(map(str, shape)) + f" {act}")
 
 
-def test_long_few_rows_keep_the_chip_busy():
-    # 64 rows of 65536 steps: with time cut into 16 runs (forward) and 32 chunks (backward) most of
-    # the chip idled for 530 and 300 us.  Bars between those and the times in chunks (60 and 140 us).
-    def timed(fn):
-        fn()
-        torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            for _ in range(4):
-                fn()
-        times = []
-        for _ in range(5):
-            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            a.record()
-            graph.replay()
-            b.record()
-            torch.cuda.synchronize()
-            times.append(a.elapsed_time(b) * 250)
-        return sorted(times)[2]
-
-    from metal_kernelops.scan import selscan_bwd_impl, selscan_fwd_impl
-    inputs, dy = _random_problem(1, 64, 65536, 16, 1, seed=5, act=torch.bfloat16)
-    args = [inputs[k].to(DEV) for k in NAMES]
-    dy = dy.to(DEV)
-    _, states = selscan_fwd_impl(*args, True)
-    assert timed(lambda: selscan_fwd_impl(*args, True)) < 300
-    assert timed(lambda: selscan_bwd_impl(dy, *args, True, states)) < 230
-
-
 @pytest.mark.parametrize("act", [torch.float32, torch.bfloat16], ids=lambda t: str(t).split(".")[-1])
 @pytest.mark.parametrize("dstate", [1, 3, 4])
 def test_narrow_states_agree_on_both_mappings(dstate, act):
